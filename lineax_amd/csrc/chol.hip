@@ -9,7 +9,7 @@
 //    keep the upper triangle resident in LDS in row-packed form (131.6 KB
 //    at n = 256): right-looking factorisation, triangular solves by one
 //    wave with the vector in registers.
-//  * larger n: one workgroup per system in global memory (correctness path).
+//  * larger n: 64-column panels over all workgroups (chol_tiled.hip).
 //
 // Failure semantics follow jax.scipy.linalg.cho_factor as lineax uses it
 // (lineax/_solver/cholesky.py:60): a non-positive or NaN pivot makes the
@@ -297,81 +297,6 @@ __global__ __launch_bounds__(kWG) void chol_solve_lds_kernel(int n, const T* __r
   }
 }
 
-// ---------------------------------------------------------------------------
-// Tier 3: any n, one workgroup per system in global memory.
-// ---------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(kWG) void chol_factor_generic_kernel(int n, T* __restrict__ a, int64_t a_stride,
-                                                                  int negate, int32_t* __restrict__ info) {
-  T* A = a + static_cast<int64_t>(blockIdx.x) * a_stride;
-  const int tid = threadIdx.x;
-  const int64_t ld = n;
-  if (negate) {
-    for (int64_t t = tid; t < ld * ld; t += kWG) {
-      const int64_t i = t / ld, j = t % ld;
-      if (j >= i) A[t] = -A[t];
-    }
-    __syncthreads();
-  }
-  int fail = 0;
-  for (int k = 0; k < n; ++k) {
-    const T akk = A[k * ld + k];
-    if (!(akk > T(0))) {
-      fail = k + 1;
-      break;
-    }
-    const T ukk = sqrt(akk);
-    for (int j = k + 1 + tid; j < n; j += kWG) A[k * ld + j] /= ukk;
-    __syncthreads();
-    if (tid == 0) A[k * ld + k] = ukk;
-    const int64_t m = n - k - 1;
-    for (int64_t t = tid; t < m * m; t += kWG) {
-      const int64_t i = k + 1 + t / m, j = k + 1 + t % m;
-      if (j >= i) A[i * ld + j] -= A[k * ld + i] * A[k * ld + j];
-    }
-    __syncthreads();
-  }
-  __syncthreads();
-  const T nan = quiet_nan<T>();
-  for (int64_t t = tid; t < ld * ld; t += kWG) {
-    const int64_t i = t / ld, j = t % ld;
-    if (fail) {
-      A[t] = nan;
-    } else if (j < i) {
-      A[t] = T(0);
-    }
-  }
-  if (tid == 0) info[blockIdx.x] = fail;
-}
-
-template <typename T>
-__global__ __launch_bounds__(kWG) void chol_solve_generic_kernel(int n, const T* __restrict__ u, int64_t u_stride,
-                                                                 T* __restrict__ b, int64_t b_stride, int negate) {
-  extern __shared__ unsigned char lxa_smem[];
-  T* v = reinterpret_cast<T*>(lxa_smem);
-  const T* U = u + static_cast<int64_t>(blockIdx.x) * u_stride;
-  T* B = b + static_cast<int64_t>(blockIdx.x) * b_stride;
-  const int tid = threadIdx.x;
-  const int64_t ld = n;
-  for (int i = tid; i < n; i += kWG) v[i] = B[i];
-  __syncthreads();
-  // U^T y = b: y_j final when read at step j; kept in B.
-  for (int j = 0; j < n; ++j) {
-    const T yj = v[j] / U[j * ld + j];
-    for (int i = j + 1 + tid; i < n; i += kWG) v[i] -= U[j * ld + i] * yj;
-    if (tid == 0) B[j] = yj;
-    __syncthreads();
-  }
-  for (int i = tid; i < n; i += kWG) v[i] = B[i];
-  __syncthreads();
-  for (int j = n - 1; j >= 0; --j) {
-    const T xj = v[j] / U[j * ld + j];
-    for (int i = tid; i < j; i += kWG) v[i] -= U[i * ld + j] * xj;
-    if (tid == 0) B[j] = negate ? -xj : xj;
-    __syncthreads();
-  }
-}
-
 // Kernels using more than 64 KiB of dynamic LDS must say so before launch.
 template <typename K>
 int allow_lds(K kernel, size_t bytes) {
@@ -419,8 +344,7 @@ int chol_factor_t(hipStream_t s, int64_t batch, int64_t n64, T* a, int64_t strid
     hipLaunchKernelGGL((chol_factor_lds_kernel<T>), dim3(static_cast<unsigned>(batch)), dim3(kWG), shmem, s, n, a,
                        stride, negate, info);
   } else {
-    hipLaunchKernelGGL((chol_factor_generic_kernel<T>), dim3(static_cast<unsigned>(batch)), dim3(kWG), 0, s, n, a,
-                       stride, negate, info);
+    return chol_tile_factor(s, batch, n, a, stride, negate, info);
   }
   LXA_LAUNCH_CHECK("lxa_chol_factor launch");
   return LXA_OK;
@@ -441,9 +365,7 @@ int chol_solve_t(hipStream_t s, int64_t batch, int64_t n64, const T* u, int64_t 
   } else {
     const size_t shmem = static_cast<size_t>(n) * sizeof(T);
     if (shmem > 160 * 1024) return set_error(LXA_EUNSUPPORTED, "lxa_chol_solve: n=%d too large", n);
-    if (int rc = allow_lds(chol_solve_generic_kernel<T>, shmem)) return rc;
-    hipLaunchKernelGGL((chol_solve_generic_kernel<T>), dim3(static_cast<unsigned>(batch)), dim3(kWG), shmem, s, n, u,
-                       us, b, bs, negate);
+    return chol_tile_solve(s, batch, n, u, us, b, bs, negate);
   }
   LXA_LAUNCH_CHECK("lxa_chol_solve launch");
   return LXA_OK;

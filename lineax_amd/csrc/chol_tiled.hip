@@ -1,0 +1,550 @@
+// Cholesky factorisation (potrf, upper: A = U^T U) of orders past the
+// one-workgroup tiers of chol.hip, in place, float32 and float64, and the
+// matching solve.
+//
+// Factor: one launch per 64-column panel, all systems of the batch and all
+// 64 x 64 tiles of the upper triangle at once.  Launch k
+//   panel tiles (k, j), j >= k: apply panel k - 1 to the diagonal tile and to
+//     tile (k, j), factor the diagonal tile (every workgroup repeats this, so
+//     no second launch and no exchange is needed) and solve U_kj with it;
+//   trailing tiles (i, j), i > k: apply panel k - 1, A_ij -= U_(k-1)i^T U_(k-1)j,
+//     on the matrix cores.
+// Panel tiles read only rows of panel k - 1, which the launch before finished;
+// the factored diagonal tile may not replace A_kk while other workgroups read
+// it, so it waits one launch in storage that nothing reads as matrix data:
+// its strictly upper part transposed in the strictly lower triangle of the
+// same tile, its diagonal in the row below that tile.
+//
+// What bounds it: the chain of n pivots (square root, reciprocal, scaling,
+// update of the next row), about 0.1 us (float) each inside a launch, plus
+// the launches.  A 16-row strip of a panel is therefore factored and solved
+// by the same instructions: lanes 0..15 of every wave hold the strip's
+// diagonal block, lanes 16..63 other columns, pivots and multipliers travel
+// by readlane and no barrier lies inside a strip.
+//
+// Reference: lineax/_solver/cholesky.py:43-78 (cho_factor / cho_solve).
+#include <algorithm>
+#include <type_traits>
+
+#include "lxa_common.h"
+
+namespace lxa {
+namespace {
+
+constexpr int kT = 64;        // tile
+constexpr int kS = 16;        // strip
+constexpr int kThreads = 256;
+constexpr int kLd = 2 * kT + 2;  // LDS row: diagonal tile, then the solved tile
+
+template <typename T>
+struct Mma;
+// One 16 x 16 x 4 matrix-core product.  Lane l: A operand [l % 16][l / 16],
+// B operand [l / 16][l % 16]; row(l, i) is the result row of register i, the
+// column is l % 16.
+template <>
+struct Mma<float> {
+  typedef float acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mul(float a, float b, acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int l, int i) { return 4 * (l >> 4) + i; }
+};
+template <>
+struct Mma<double> {
+  typedef double acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mul(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int l, int i) { return (l >> 4) + 4 * i; }
+};
+
+__device__ __forceinline__ float from_lane(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ double from_lane(double v, int lane) {
+  const int64_t bits = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane(static_cast<int>(bits & 0xffffffff), lane);
+  const int hi = __builtin_amdgcn_readlane(static_cast<int>(bits >> 32), lane);
+  return __longlong_as_double((static_cast<int64_t>(hi) << 32) | static_cast<uint32_t>(lo));
+}
+
+template <int B, int E, typename F>
+__device__ __forceinline__ void unroll(F&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    unroll<B + 1, E>(f);
+  }
+}
+
+// Rows k0 .. k0 + 63 of the factor, columns c0 .. c0 + 63, to LDS columns
+// at .. at + 63 of P; zero past column n (rows k0 .. k0 + 63 all exist).
+template <typename T>
+__device__ __forceinline__ void load_rows(const T* A, int64_t ld, int n, int k0, int c0, T* P, int at) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int col = c0 + lane, cc = min(col, n - 1);
+  T v[kT / 4];
+#pragma unroll
+  for (int u = 0; u < kT / 4; ++u) v[u] = A[(int64_t)(k0 + wv + 4 * u) * ld + cc];
+#pragma unroll
+  for (int u = 0; u < kT / 4; ++u) P[(wv + 4 * u) * kLd + at + lane] = col < n ? v[u] : T(0);
+}
+
+// Launch k of the factorisation; nt tiles per side.  Workgroups [0, batch *
+// (nt - k)) are the panel tiles, the rest the trailing tiles.
+template <typename T>
+__global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_kernel(int64_t batch, int n, int k, int nt, T* __restrict__ a,
+                                                             int64_t a_stride, int negate,
+                                                             int32_t* __restrict__ info) {
+  using M4 = typename Mma<T>::acc;
+  extern __shared__ __align__(16) unsigned char lxa_smem[];
+  T* P = reinterpret_cast<T*>(lxa_smem);  // [64][kLd]: rows of panel k - 1
+  T* M = P + kT * kLd;                    // [64][kLd]: diagonal tile and tile (k, j)
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int q = lane & 15, g = lane >> 4;
+  const int64_t sys = blockIdx.x % batch;
+  int t = (int)(blockIdx.x / batch);
+  T* A = a + sys * a_stride;
+  const int64_t ld = n;
+  const int k0 = k * kT;
+  // the matrix itself is read for the first time by launch 0 (row 0 of tiles)
+  // and launch 1 (all others)
+  const T sign = (negate && k <= 1) ? T(-1) : T(1);
+
+  if (t >= nt - k) {
+    // ---- trailing tile (i, j), k < i <= j
+    t -= nt - k;
+    int i = k + 1;
+    while (t >= nt - i) {
+      t -= nt - i;
+      ++i;
+    }
+    const int j = i + t;
+    load_rows(A, ld, n, k0 - kT, i * kT, P, 0);
+    load_rows(A, ld, n, k0 - kT, j * kT, P, kT);
+    M4 acc[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int col = min(j * kT + 16 * c + q, n - 1);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        // clamped onto the upper triangle; entries outside are not stored
+        const int row = min(i * kT + 16 * wv + Mma<T>::row(lane, e), col);
+        acc[c][e] = sign * A[(int64_t)row * ld + col];
+      }
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int s = 0; s < kT; s += 4) {
+      const T* Ps = P + (s + g) * kLd;
+      const T av = -Ps[16 * wv + q];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] = Mma<T>::mul(av, Ps[kT + 16 * c + q], acc[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int col = j * kT + 16 * c + q;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = i * kT + 16 * wv + Mma<T>::row(lane, e);
+        if (col < n && row <= col) A[(int64_t)row * ld + col] = acc[c][e];
+      }
+    }
+    return;
+  }
+
+  // ---- panel tile (k, j): M = [A_kk | A_kj] with panel k - 1 applied
+  const int j = k + t;
+  const int kb = min(kT, n - k0);
+  const int ctiles = j > k ? 8 : 4;
+  if (k > 0) {
+    load_rows(A, ld, n, k0 - kT, k0, P, 0);
+    if (j > k) load_rows(A, ld, n, k0 - kT, j * kT, P, kT);
+  }
+  {
+    M4 acc[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      if (c >= ctiles || (c < 4 && c < wv)) continue;  // uniform
+      const int cl = 16 * (c & 3) + q;
+      const int col = (c < 4 ? k0 : j * kT) + cl, cc = min(col, n - 1);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 16 * wv + Mma<T>::row(lane, e);
+        const T v = sign * A[(int64_t)min(k0 + r, cc) * ld + cc];
+        const bool in = c < 4 ? (r <= cl && cl < kb) : col < n;
+        // past the last row the diagonal tile continues as the identity
+        acc[c][e] = in ? v : (c < 4 && r == cl) ? T(1) : T(0);
+      }
+    }
+    __syncthreads();
+    if (k > 0) {
+#pragma unroll 2
+      for (int s = 0; s < kT; s += 4) {
+        const T* Ps = P + (s + g) * kLd;
+        const T av = -Ps[16 * wv + q];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          if (c >= ctiles || (c < 4 && c < wv)) continue;
+          acc[c] = Mma<T>::mul(av, Ps[16 * c + q], acc[c]);
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      if (c >= ctiles || (c < 4 && c < wv)) continue;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) M[(16 * wv + Mma<T>::row(lane, e)) * kLd + 16 * c + q] = acc[c][e];
+    }
+  }
+  __syncthreads();
+
+  int fail = 0;
+#pragma unroll 1
+  for (int s = 0; s < kT / kS; ++s) {
+    // ---- strip s: lanes 0..15 of each wave hold its diagonal block, lanes
+    // 16..63 the wave's share of the columns right of it
+    const int r0 = s * kS;
+    const int others = 16 * ctiles - r0 - kS;
+    const int oc = wv * 48 + lane - kS;
+    const int col = lane < kS ? r0 + lane : r0 + kS + min(oc, others - 1);
+    const bool mine = lane < kS ? wv == 0 : oc < others;
+    if (wv == 0 || wv * 48 < others) {  // uniform
+      // opaque per strip: the 16 lane masks are formed where they are used
+      // instead of being held, and spilled, across the strips
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      T c[kS];
+      T* Ms = M + r0 * kLd + (others > 0 ? col : min(col, r0 + kS - 1));
+#pragma unroll
+      for (int i = 0; i < kS; ++i) c[i] = Ms[i * kLd];
+      unroll<0, kS>([&](auto T_) __attribute__((always_inline)) {
+        constexpr int p = decltype(T_)::value;
+        const T d = from_lane(c[p], p);
+        if (!(d > T(0)) && fail == 0) fail = k0 + r0 + p + 1;
+        const T u = sqrt(d);  // NaN for a negative pivot
+        const T inv = T(1) / u;
+        c[p] = ln == p ? u : c[p] * inv;
+        unroll<p + 1, kS>([&](auto I_) __attribute__((always_inline)) {
+          constexpr int i = decltype(I_)::value;
+          c[i] -= from_lane(c[p], i) * c[p];
+        });
+      });
+      if (mine) {
+#pragma unroll
+        for (int i = 0; i < kS; ++i) Ms[i * kLd] = c[i];
+      }
+    }
+    __syncthreads();
+    // ---- the rows below: M_rc -= M_sr^T M_sc, 16 x 16 tiles dealt to the
+    // waves (row strip r, column tile c >= r)
+    int idx = wv;
+#pragma unroll 1
+    for (int r = s + 1; r < 4; ++r) {
+      const int cnt = ctiles - r;
+#pragma unroll 1
+      for (; idx < cnt; idx += 4) {
+        const int c = r + idx;
+        M4 acc;
+        T* Mt = M + 16 * r * kLd + 16 * c + q;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = Mt[Mma<T>::row(lane, e) * kLd];
+#pragma unroll
+        for (int h = 0; h < kS; h += 4) {
+          const T* Mh = M + (r0 + h + g) * kLd;
+          acc = Mma<T>::mul(-Mh[16 * r + q], Mh[16 * c + q], acc);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) Mt[Mma<T>::row(lane, e) * kLd] = acc[e];
+      }
+      idx -= cnt;
+    }
+    __syncthreads();
+  }
+
+  if (j > k) {
+    // U_kj (all 64 rows exist), and zeros below the diagonal in tile (j, k);
+    // row 0 of tile (k + 1, k) holds the diagonal of U_kk until the next launch
+    const int col = j * kT + lane;
+    for (int r = wv; r < kT; r += 4) {
+      if (col < n) A[(int64_t)(k0 + r) * ld + col] = M[r * kLd + kT + lane];
+      const int zr = j * kT + r;
+      if (zr < n && !(j == k + 1 && r == 0)) A[(int64_t)zr * ld + k0 + lane] = T(0);
+    }
+    return;
+  }
+  if (k > 0) {
+    // the diagonal tile of the launch before moves to its place
+    const int p0 = k0 - kT;
+    for (int e = tid; e < kT * kT; e += kThreads) {
+      const int r = e / kT, c = e % kT;
+      if (r < c) P[r * kLd + c] = A[(int64_t)(p0 + c) * ld + p0 + r];
+      if (r == c) P[r * kLd + c] = A[(int64_t)k0 * ld + p0 + c];
+      if (r > c) P[r * kLd + c] = T(0);
+    }
+    __syncthreads();  // every stored value is read before it is overwritten
+    for (int e = tid; e < kT * kT; e += kThreads) {
+      const int r = e / kT, c = e % kT;
+      A[(int64_t)(p0 + r) * ld + p0 + c] = P[r * kLd + c];
+    }
+    if (tid < kT) A[(int64_t)k0 * ld + p0 + tid] = T(0);
+  }
+  const bool last = k == nt - 1;
+  for (int e = tid; e < kT * kT; e += kThreads) {
+    const int r = e / kT, c = e % kT;
+    if (r >= kb || c >= kb) continue;
+    if (last) {
+      A[(int64_t)(k0 + r) * ld + k0 + c] = r <= c ? M[r * kLd + c] : T(0);
+    } else if (r > c) {
+      A[(int64_t)(k0 + r) * ld + k0 + c] = M[c * kLd + r];
+    } else if (r == c) {
+      A[(int64_t)(k0 + kT) * ld + k0 + c] = M[r * kLd + c];
+    }
+  }
+  if (tid == 0 && (k == 0 || (fail && info[sys] == 0))) info[sys] = fail;
+}
+
+// The whole factor of a system that failed becomes NaN.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void chol_fail_kernel(int n, T* __restrict__ a, int64_t a_stride,
+                                                             const int32_t* __restrict__ info, int64_t sys0) {
+  const int64_t sys = sys0 + blockIdx.x;
+  if (info[sys] == 0) return;
+  T* A = a + sys * a_stride;
+  const int64_t nn = (int64_t)n * n;
+  for (int64_t e = threadIdx.x; e < nn; e += kThreads) A[e] = quiet_nan<T>();
+}
+
+// ---------------------------------------------------------------------------
+// U^T U x = b, one right-hand side per system, one 1024-thread workgroup each.
+// Thread t holds columns t, t + 1024, ... of the vector in LDS and reads rows
+// of U (coalesced) in both directions:
+//   forward   y_j -= sum over the block's rows i of U_ij y_i, right-looking;
+//   backward  sum over columns j of U_ij x_j for the block's rows, left-looking,
+//             a wave reduce-scatter and a sum over waves in a fixed order.
+// The kRows x 1 values a thread needs for its first column of the next block
+// are loaded before the current block's chain of divisions starts, so that
+// the loads' latency is hidden by it.  That chain (kRows steps by one wave,
+// multipliers in registers) bounds the solve.
+// ---------------------------------------------------------------------------
+constexpr int kSolveThreads = 1024;
+constexpr int kSolveWaves = kSolveThreads / kWave;
+
+template <typename T>
+struct SolveRows {
+  static constexpr int value = sizeof(T) == 4 ? 32 : 16;
+};
+
+template <typename T, bool InLds>
+__global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, const T* __restrict__ u,
+                                                                        int64_t u_stride, T* __restrict__ b,
+                                                                        int64_t b_stride, int negate) {
+  constexpr int R = SolveRows<T>::value;
+  extern __shared__ __align__(16) unsigned char lxa_smem[];
+  T* ys = reinterpret_cast<T*>(lxa_smem);  // [n rounded up to R]
+  __shared__ T part[kSolveWaves][R];
+  __shared__ T D[2][R][R + 1];            // diagonal blocks, double-buffered
+  __shared__ T rd[2][R];                  // reciprocals of their diagonals
+  const T* U = u + (int64_t)blockIdx.x * u_stride;
+  T* B = b + (int64_t)blockIdx.x * b_stride;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int64_t ld = n;
+  const int blocks = (n + R - 1) / R;
+  // the vector: in LDS, or in place in global memory where it would not fit
+  // beside the buffers above
+  auto get = [&](int i) -> T {
+    if constexpr (InLds) return ys[i];
+    return i < n ? B[i] : T(0);
+  };
+  auto put = [&](int i, T x) {
+    if constexpr (InLds) {
+      ys[i] = x;
+    } else {
+      if (i < n) B[i] = x;
+    }
+  };
+  if constexpr (InLds) {
+    for (int i = tid; i < blocks * R; i += kSolveThreads) ys[i] = i < n ? B[i] : T(0);
+  }
+
+  // threads 0 .. R * R - 1 carry the diagonal block of block p through here
+  T dv = T(0);
+  const int di = tid / R, dj = tid % R;
+  auto fetch_diag = [&](int p) {
+    if (tid < R * R) {
+      const int j = min(p * R + dj, n - 1);
+      dv = U[(int64_t)min(p * R + di, j) * ld + j];
+    }
+  };
+  auto stash_diag = [&](int p) {
+    if (tid < R * R) {
+      const bool in = p * R + dj < n && dj >= di;
+      D[p & 1][di][dj] = in ? dv : T(0);
+      if (di == dj) rd[p & 1][di] = in ? T(1) / dv : T(0);  // padding solves to 0
+    }
+  };
+  // column c, the R rows of block p (rows clamped; clamped ones meet y = 0)
+  T v[R];
+  auto fetch = [&](int p, int c) {
+    const int cc = min(c, n - 1);
+#pragma unroll
+    for (int i = 0; i < R; ++i) v[i] = U[(int64_t)min(p * R + i, n - 1) * ld + cc];
+  };
+
+  // ---- U^T y = b
+  fetch_diag(0);
+  stash_diag(0);
+  __syncthreads();
+  for (int p = 0; p < blocks; ++p) {
+    const int c0 = p * R + R;
+    fetch(p, c0 + tid);
+    if (p + 1 < blocks) fetch_diag(p + 1);
+    if (wv == 0) {
+      T z = lane < R ? get(p * R + lane) : T(0);
+      int ln = lane;  // opaque per block: lane masks are not held across blocks
+      asm volatile("" : "+v"(ln));
+      const T r = lane < R ? rd[p & 1][lane] : T(0);
+      T m[R];
+#pragma unroll
+      for (int i = 0; i < R; ++i) m[i] = lane < R ? D[p & 1][i][lane] : T(0);
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        if (ln == i) z *= r;
+        const T zi = from_lane(z, i);
+        if (ln > i) z -= m[i] * zi;
+      }
+      if (lane < R) put(p * R + lane, z);
+    }
+    __syncthreads();
+    if (p + 1 < blocks) stash_diag(p + 1);
+    for (int c = c0 + tid; c < n; c += kSolveThreads) {
+      if (c >= c0 + kSolveThreads) fetch(p, c);
+      T s = T(0);
+#pragma unroll
+      for (int i = 0; i < R; ++i) s += v[i] * get(p * R + i);
+      put(c, get(c) - s);
+    }
+    __syncthreads();
+  }
+
+  // ---- U x = y
+  fetch_diag(blocks - 1);
+  stash_diag(blocks - 1);
+  if (tid < kSolveWaves * R) part[tid / R][tid % R] = T(0);
+  __syncthreads();
+  for (int p = blocks - 1; p >= 0; --p) {
+    // the products with the columns solved so far, except those of the block
+    // solved last, are in part; this block's rows of those columns follow
+    if (p > 0) {
+      fetch_diag(p - 1);
+      fetch(p - 1, p * R + tid);
+    }
+    if (wv == 0) {
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      T z = T(0);
+      if (lane < R) {
+        z = get(p * R + lane);
+        T s = T(0);
+#pragma unroll
+        for (int w = 0; w < kSolveWaves; ++w) s += part[w][lane];
+        z -= s;
+      }
+      const T r = lane < R ? rd[p & 1][lane] : T(0);
+      T m[R];
+#pragma unroll
+      for (int i = 0; i < R; ++i) m[i] = lane < R ? D[p & 1][lane][i] : T(0);
+#pragma unroll
+      for (int i = R - 1; i >= 0; --i) {
+        if (ln == i) z *= r;
+        const T zi = from_lane(z, i);
+        if (ln < i) z -= m[i] * zi;
+      }
+      if (lane < R) put(p * R + lane, z);
+    }
+    __syncthreads();
+    if (p > 0) {
+      stash_diag(p - 1);
+      T s[R];
+#pragma unroll
+      for (int i = 0; i < R; ++i) s[i] = T(0);
+      const int c0 = p * R;
+      for (int c = c0 + tid; c < n; c += kSolveThreads) {
+        if (c >= c0 + kSolveThreads) fetch(p - 1, c);
+        const T x = get(c);
+#pragma unroll
+        for (int i = 0; i < R; ++i) s[i] += v[i] * x;
+      }
+      if (c0 + wv * kWave < n || p == blocks - 1) {
+        const T t = wave_reduce_scatter<R>(s, lane);
+        constexpr int kShift = 6 - Log2<R>::value;
+        if ((lane & ((1 << kShift) - 1)) == 0) part[wv][lane >> kShift] = t;
+      }
+    }
+    __syncthreads();
+  }
+  for (int i = tid; i < n; i += kSolveThreads) {
+    const T x = get(i);
+    B[i] = negate ? -x : x;
+  }
+}
+
+template <typename T>
+int factor_t(hipStream_t st, int64_t batch, int n, T* a, int64_t stride, int negate, int32_t* info) {
+  const size_t smem = sizeof(T) * 2 * kT * kLd;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&chol_tile_kernel<T>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+  if (e != hipSuccess) return hip_error(e, "hipFuncSetAttribute(chol_tile_kernel)");
+  const int nt = (n + kT - 1) / kT;
+  const int64_t most = (int64_t)nt + (int64_t)nt * (nt - 1) / 2;  // tiles of launch 1, the widest, or of launch 0
+  // a grid holds fewer than 2^32 threads
+  const int64_t chunk = std::max<int64_t>(1, (int64_t(1) << 23) / most);
+  for (int64_t s0 = 0; s0 < batch; s0 += chunk) {
+    const int64_t cnt = std::min(chunk, batch - s0);
+    for (int k = 0; k < nt; ++k) {
+      const int64_t rest = nt - k - 1;
+      const int64_t tiles = nt - k + (k > 0 ? rest * (rest + 1) / 2 : 0);
+      chol_tile_kernel<T><<<dim3((unsigned)(tiles * cnt)), kThreads, smem, st>>>(cnt, n, k, nt, a + s0 * stride, stride,
+                                                                                  negate, info + s0);
+    }
+    chol_fail_kernel<T><<<dim3((unsigned)cnt), kThreads, 0, st>>>(n, a, stride, info, s0);
+  }
+  LXA_LAUNCH_CHECK("chol_tile_kernel");
+  return LXA_OK;
+}
+
+template <typename T, bool InLds>
+int solve_launch(hipStream_t st, int64_t batch, int n, const T* u, int64_t us, T* b, int64_t bs, int negate) {
+  constexpr int R = SolveRows<T>::value;
+  const size_t smem = InLds ? sizeof(T) * (size_t)((n + R - 1) / R * R) : 0;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&chol_tile_solve_kernel<T, InLds>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+  if (e != hipSuccess) return hip_error(e, "hipFuncSetAttribute(chol_tile_solve_kernel)");
+  chol_tile_solve_kernel<T, InLds><<<dim3((unsigned)batch), kSolveThreads, smem, st>>>(n, u, us, b, bs, negate);
+  LXA_LAUNCH_CHECK("chol_tile_solve_kernel");
+  return LXA_OK;
+}
+
+template <typename T>
+int solve_t(hipStream_t st, int64_t batch, int n, const T* u, int64_t us, T* b, int64_t bs, int negate) {
+  if (sizeof(T) * (size_t)n <= 128 * 1024) return solve_launch<T, true>(st, batch, n, u, us, b, bs, negate);
+  return solve_launch<T, false>(st, batch, n, u, us, b, bs, negate);
+}
+
+}  // namespace
+
+int chol_tile_factor(hipStream_t s, int64_t batch, int n, float* a, int64_t stride, int negate, int32_t* info) {
+  return factor_t<float>(s, batch, n, a, stride, negate, info);
+}
+int chol_tile_factor(hipStream_t s, int64_t batch, int n, double* a, int64_t stride, int negate, int32_t* info) {
+  return factor_t<double>(s, batch, n, a, stride, negate, info);
+}
+int chol_tile_solve(hipStream_t s, int64_t batch, int n, const float* u, int64_t us, float* b, int64_t bs,
+                    int negate) {
+  return solve_t<float>(s, batch, n, u, us, b, bs, negate);
+}
+int chol_tile_solve(hipStream_t s, int64_t batch, int n, const double* u, int64_t us, double* b, int64_t bs,
+                    int negate) {
+  return solve_t<double>(s, batch, n, u, us, b, bs, negate);
+}
+
+}  // namespace lxa

@@ -173,6 +173,14 @@ __device__ __forceinline__ int packed_upper(int n, int i, int j) {
 // lxa_chol_factor.
 int chol_factor_regs_f32(hipStream_t s, int64_t batch, int n, float* a, int64_t stride, int negate, int32_t* info);
 
+// Cholesky factor and solve of orders past the one-workgroup tiers
+// (chol_tiled.hip); conventions of lxa_chol_factor / lxa_chol_solve.
+int chol_tile_factor(hipStream_t s, int64_t batch, int n, float* a, int64_t stride, int negate, int32_t* info);
+int chol_tile_factor(hipStream_t s, int64_t batch, int n, double* a, int64_t stride, int negate, int32_t* info);
+int chol_tile_solve(hipStream_t s, int64_t batch, int n, const float* u, int64_t us, float* b, int64_t bs, int negate);
+int chol_tile_solve(hipStream_t s, int64_t batch, int n, const double* u, int64_t us, double* b, int64_t bs,
+                    int negate);
+
 }  // namespace lxa
 
 #define LXA_REQUIRE(cond, ...)                                   \

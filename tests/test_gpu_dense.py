@@ -171,6 +171,50 @@ def test_cholesky_reads_upper_triangle_only(device, rng, n, dtype):
     assert torch.equal(u1, u2)
 
 
+@pytest.mark.parametrize("n,dtype", [
+    (257, torch.float32), (319, torch.float32), (320, torch.float32), (321, torch.float32), (577, torch.float32),
+    (182, torch.float64), (192, torch.float64), (193, torch.float64), (256, torch.float64), (449, torch.float64),
+    (1100, torch.float64),
+])
+def test_cholesky_tiled(device, rng, n, dtype):
+    """Orders around the 64-row tiles, past 1024 columns (two per thread in the
+    solve), either sign, garbage below the diagonal, a batch of which one fails.
+
+    Bounds: |U^T U - A| <= gamma_(n+1) |U|^T |U| componentwise (Higham, Accuracy
+    and Stability, thm 10.3; the row norms of |U|^T |U| are below max a_ii), and
+    (3 n + 1) u on the backward error of the solve (thm 10.4), doubled for the
+    reciprocal pivots."""
+    eps = torch.finfo(dtype).eps / 2
+    for negate in (False, True):
+        sign = -1.0 if negate else 1.0
+        mats = [well_conditioned(rng, n, kind="psd") for _ in range(2)]
+        given = []
+        for a in mats:
+            g = sign * a
+            g[np.tril_indices(n, -1)] = 1e30
+            given.append(g)
+        bad = given[1].copy()
+        bad[n - 2, n - 2] *= -1.0
+        early = given[1].copy()
+        early[3, 3] *= -1.0
+        t = _t(np.stack(given + [bad, early]), device, dtype)
+        u, info = K.chol_factor(t, negate=negate)
+        assert info.tolist() == [0, 0, n - 1, 4]
+        assert bool(torch.isnan(u[2:]).all())
+        rhs = _t(rng.standard_normal((4, n)), device, dtype)
+        x = K.chol_solve(u, rhs, negate=negate).cpu().double()
+        assert bool(torch.isnan(x[2:]).all())
+        exact = torch.triu(t[:2].cpu().double())
+        exact = exact + torch.triu(exact, 1).mT
+        uc = u[:2].cpu().double()
+        assert bool((torch.tril(uc, -1) == 0).all())
+        resid = (uc.mT @ uc - sign * exact).abs()
+        assert bool((resid <= 2 * (n + 2) * eps * (uc.abs().mT @ uc.abs())).all())
+        r = (exact @ x[:2, :, None])[..., 0] - rhs[:2].cpu().double()
+        scale = (uc.abs().mT @ (uc.abs() @ x[:2, :, None].abs()))[..., 0]
+        assert bool((r.abs() <= 2 * (3 * n + 2) * eps * scale).all())
+
+
 def test_gemv_matches(device, rng):
     # (5000, 300) and (4099, 37) split the transposed product over row chunks
     # (the 16-byte path and the scalar path); the rest run in one chunk
