@@ -9,9 +9,11 @@
 // result (LU in place plus 0-based interchange sequence) is exactly
 // LAPACK's getrf output format, so jax.scipy's lu_solve semantics apply.
 //
+// Orders 65..256 take the blocked one-workgroup kernels of lu_mid.hip.
+//
 // Larger orders use a one-workgroup-per-system right-looking kernel working
-// in global memory (correctness path for moderate n; single large float32
-// systems take the blocked path of lu_large.hip and gemm.hip instead).
+// in global memory (correctness path; up to 16 large systems take the blocked
+// path of lu_large.hip and gemm.hip instead).
 #include <climits>
 
 #include "lxa_common.h"
@@ -421,12 +423,15 @@ void dispatch_solve_small(int n, hipStream_t s, int64_t batch, const T* lu, int6
 }
 
 constexpr int kSmallMax = 64;
+constexpr int kMidMax = 256;  // lu_mid.hip: one thread per unknown, four rows per lane of its panel wave
 constexpr int64_t kMaxGrid = 2147483647;
 
 template <typename T>
 int lu_factor_t(hipStream_t s, int64_t batch, int64_t n, T* a, int64_t stride, int32_t* piv, int32_t* info) {
   if (n <= kSmallMax) {
     dispatch_factor_small<T>(static_cast<int>(n), s, batch, a, stride, piv, info);
+  } else if (n <= kMidMax) {
+    return lu_mid_factor(s, batch, static_cast<int>(n), a, stride, piv, info);
   } else {
     hipLaunchKernelGGL((lu_factor_generic_kernel<T>), dim3(static_cast<unsigned>(batch)), dim3(256), 0, s,
                        static_cast<int>(n), a, stride, piv, info);
@@ -440,6 +445,8 @@ int lu_solve_t(hipStream_t s, int64_t batch, int64_t n, const T* lu, int64_t lus
                int64_t ps, T* b, int64_t bs, int trans) {
   if (n <= kSmallMax) {
     dispatch_solve_small<T>(static_cast<int>(n), s, batch, lu, lus, piv, ps, b, bs, trans);
+  } else if (n <= kMidMax) {
+    return lu_mid_solve(s, batch, static_cast<int>(n), lu, lus, piv, ps, b, bs, trans);
   } else {
     const size_t shmem = static_cast<size_t>(n) * sizeof(T);
     if (shmem > 160 * 1024) return set_error(LXA_EUNSUPPORTED, "lxa_lu_solve: n=%lld too large", (long long)n);

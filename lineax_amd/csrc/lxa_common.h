@@ -181,6 +181,15 @@ int chol_tile_solve(hipStream_t s, int64_t batch, int n, const float* u, int64_t
 int chol_tile_solve(hipStream_t s, int64_t batch, int n, const double* u, int64_t us, double* b, int64_t bs,
                     int negate);
 
+// Batched getrf / getrs of orders 65..256 (lu_mid.hip); conventions of
+// lxa_lu_factor / lxa_lu_solve.
+int lu_mid_factor(hipStream_t s, int64_t batch, int n, float* a, int64_t stride, int32_t* piv, int32_t* info);
+int lu_mid_factor(hipStream_t s, int64_t batch, int n, double* a, int64_t stride, int32_t* piv, int32_t* info);
+int lu_mid_solve(hipStream_t s, int64_t batch, int n, const float* lu, int64_t lus, const int32_t* piv, int64_t ps,
+                 float* b, int64_t bs, int trans);
+int lu_mid_solve(hipStream_t s, int64_t batch, int n, const double* lu, int64_t lus, const int32_t* piv, int64_t ps,
+                 double* b, int64_t bs, int trans);
+
 }  // namespace lxa
 
 #define LXA_REQUIRE(cond, ...)                                   \

@@ -50,6 +50,54 @@ def test_lu_solve_f64(device, rng, n, trans):
         np.testing.assert_allclose(x[i], ref, rtol=1e-10, atol=1e-10)
 
 
+@pytest.mark.parametrize("n,dtype", [
+    (65, torch.float32), (128, torch.float32), (129, torch.float32), (192, torch.float32), (199, torch.float32),
+    (200, torch.float32), (255, torch.float32), (256, torch.float32),
+    (66, torch.float64), (128, torch.float64), (141, torch.float64), (142, torch.float64), (193, torch.float64),
+    (256, torch.float64),
+])
+def test_lu_mid(device, rng, n, dtype):
+    """Orders around the panel, register-slot and LDS limits of the blocked
+    kernels; pivot ties, a zero column, both transposes.
+
+    Bounds: |P A - L U| <= gamma_n |L| |U| and |b - op(A) x| <= gamma_(3n) |L| |U| |x|
+    (P^T applied) componentwise (Higham, Accuracy and Stability, thm 9.3 and
+    9.4), gamma doubled for the corrected reciprocals in place of divisions."""
+    eps = torch.finfo(dtype).eps / 2
+    mats = np.stack([well_conditioned(rng, n), np.sign(rng.standard_normal((n, n))) + n * np.eye(n)[::-1],
+                     well_conditioned(rng, n)])
+    mats[2, :, n // 2] = 0.0
+    mats[1, :, 0] = np.where(rng.random(n) < 0.5, 3.0, -3.0)  # every row ties for the first pivot
+    t = _t(mats, device, dtype)
+    lu, piv, info = K.lu_factor(t)
+    assert info.tolist() == [0, 0, n // 2 + 1]
+    assert piv[1, 0] == 0
+    if dtype == torch.float64:
+        np.testing.assert_array_equal(piv[0].cpu().numpy(), O.lu_factor(mats[0])[1])
+    lc = lu.double().cpu()
+    L = torch.tril(lc, -1) + torch.eye(n, dtype=torch.float64)
+    U = torch.triu(lc)
+    assert bool((L.abs() <= 1 + 4 * eps).all())
+    exact = t.double().cpu()
+    perm = torch.arange(n).repeat(3, 1)
+    for i, row in enumerate(piv.tolist()):
+        for k, p in enumerate(row):
+            perm[i, [k, p]] = perm[i, [p, k]]
+    pa = torch.stack([exact[i][perm[i]] for i in range(3)])
+    assert bool(((pa - L @ U).abs() <= 2 * (n + 1) * eps * (L.abs() @ U.abs())).all())
+    rhs = _t(rng.standard_normal((3, n)), device, dtype)
+    absolute = torch.empty_like(pa)
+    for i in range(3):
+        absolute[i][perm[i]] = (L.abs() @ U.abs())[i]
+    for trans in (0, 1):
+        x = K.lu_solve(lu, piv, rhs, trans).double().cpu()
+        assert not bool(torch.isfinite(x[2]).all())
+        op, bound = (exact.mT, absolute.mT) if trans else (exact, absolute)
+        r = (rhs.double().cpu() - (op @ x[..., None])[..., 0]).abs()
+        lim = 2 * (3 * n + 2) * eps * (bound @ x.abs()[..., None])[..., 0]
+        assert bool((r[:2] <= lim[:2]).all())
+
+
 def test_small_lu_config_batch_f32(device):
     # The 1024 x (32 x 32) configuration: pivots equal the oracle's and the
     # float32 solutions are backward stable against the exact data.
