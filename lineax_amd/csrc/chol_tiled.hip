@@ -76,17 +76,56 @@ __device__ __forceinline__ void unroll(F&& f) {
   }
 }
 
-// Rows k0 .. k0 + 63 of the factor, columns c0 .. c0 + 63, to LDS columns
-// at .. at + 63 of P; zero past column n (rows k0 .. k0 + 63 all exist).
+// Square root and its reciprocal of a pivot, from the hardware reciprocal
+// square root and Newton steps (the correctly rounded sqrt and division cost
+// about four times as many dependent instructions on the chain): within an
+// ulp or two of both.
+__device__ __forceinline__ void pivot_root(float d, float& u, float& inv) {
+  float r = __builtin_amdgcn_rsqf(d);
+  r = fmaf(r, fmaf(-d * r, 0.5f * r, 0.5f), r);
+  u = d * r;
+  u = fmaf(fmaf(-u, u, d), 0.5f * r, u);
+  inv = r;
+}
+__device__ __forceinline__ void pivot_root(double d, double& u, double& inv) {
+  double r = __builtin_amdgcn_rsq(d);
+  r = fma(r, fma(-d * r, 0.5 * r, 0.5), r);
+  r = fma(r, fma(-d * r, 0.5 * r, 0.5), r);
+  u = d * r;
+  u = fma(fma(-u, u, d), 0.5 * r, u);
+  inv = r;
+}
+// Pivots for which every step above stays normal.
+__device__ __forceinline__ bool root_range(float d) { return d >= 0x1p-80f && d <= 0x1p80f; }
+__device__ __forceinline__ bool root_range(double d) { return d >= 0x1p-800 && d <= 0x1p800; }
+
+// Rows k0 .. k0 + 63 of the factor (all exist), columns c0 .. c0 + 63 (zero
+// past column n): to registers, then to LDS columns at .. at + 63 of P, so
+// that all of a workgroup's loads can be issued before any is waited for.
+constexpr int kRowsPer = kT / (kThreads / kWave);
 template <typename T>
-__device__ __forceinline__ void load_rows(const T* A, int64_t ld, int n, int k0, int c0, T* P, int at) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int col = c0 + lane, cc = min(col, n - 1);
-  T v[kT / 4];
+__device__ __forceinline__ void fetch_rows(const T* A, int64_t ld, int n, int k0, int c0, T (&v)[kRowsPer]) {
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned cc = min(c0 + lane, n - 1);
+  const T* p = A + (int64_t)(k0 + wv) * ld;  // uniform: stepped on the scalar unit
 #pragma unroll
-  for (int u = 0; u < kT / 4; ++u) v[u] = A[(int64_t)(k0 + wv + 4 * u) * ld + cc];
+  for (int u = 0; u < kRowsPer; ++u, p += 4 * ld) v[u] = p[cc];
+}
+template <typename T>
+__device__ __forceinline__ void stash_rows(const T (&v)[kRowsPer], int n, int c0, T* P, int at) {
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
-  for (int u = 0; u < kT / 4; ++u) P[(wv + 4 * u) * kLd + at + lane] = col < n ? v[u] : T(0);
+  for (int u = 0; u < kRowsPer; ++u) P[(wv + 4 * u) * kLd + at + lane] = c0 + lane < n ? v[u] : T(0);
+}
+
+// Advances p by `steps` rows, but not past row n - 1 (row: p's row).  Row
+// addresses are stepped instead of multiplied out: a 64-bit product per
+// load costs more issue slots than the rest of the tile's arithmetic.
+template <typename P>
+__device__ __forceinline__ void step_rows(P& p, int& row, int steps, int n, int64_t ld) {
+  const int to = min(row + steps, n - 1);
+  p += (to - row == steps) ? steps * ld : (int64_t)(to - row) * ld;
+  row = to;
 }
 
 // Launch k of the factorisation; nt tiles per side.  Workgroups [0, batch *
@@ -99,7 +138,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
   extern __shared__ __align__(16) unsigned char lxa_smem[];
   T* P = reinterpret_cast<T*>(lxa_smem);  // [64][kLd]: rows of panel k - 1
   T* M = P + kT * kLd;                    // [64][kLd]: diagonal tile and tile (k, j)
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q = lane & 15, g = lane >> 4;
   const int64_t sys = blockIdx.x % batch;
   int t = (int)(blockIdx.x / batch);
@@ -119,19 +158,24 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
       ++i;
     }
     const int j = i + t;
-    load_rows(A, ld, n, k0 - kT, i * kT, P, 0);
-    load_rows(A, ld, n, k0 - kT, j * kT, P, kT);
+    T vi[kRowsPer], vj[kRowsPer];
+    fetch_rows(A, ld, n, k0 - kT, i * kT, vi);
+    fetch_rows(A, ld, n, k0 - kT, j * kT, vj);
     M4 acc[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int col = min(j * kT + 16 * c + q, n - 1);
+    {
+      int row = min(i * kT + 16 * wv + Mma<T>::row(lane, 0), n - 1);
+      const T* p = A + (int64_t)row * ld;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        // clamped onto the upper triangle; entries outside are not stored
-        const int row = min(i * kT + 16 * wv + Mma<T>::row(lane, e), col);
-        acc[c][e] = sign * A[(int64_t)row * ld + col];
+        // entries below the diagonal (tile i = j) are loaded and not stored
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[c][e] = sign * p[min(j * kT + 16 * c + q, n - 1)];
+        if (e < 3) step_rows(p, row, Mma<T>::row(0, e + 1) - Mma<T>::row(0, e), n, ld);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the stores
+    stash_rows(vi, n, i * kT, P, 0);
+    stash_rows(vj, n, j * kT, P, kT);
     __syncthreads();
 #pragma unroll 2
     for (int s = 0; s < kT; s += 4) {
@@ -140,13 +184,21 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
 #pragma unroll
       for (int c = 0; c < 4; ++c) acc[c] = Mma<T>::mul(av, Ps[kT + 16 * c + q], acc[c]);
     }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int col = j * kT + 16 * c + q;
+    {
+      int row = i * kT + 16 * wv + Mma<T>::row(lane, 0);
+      T* p = A + (int64_t)row * ld;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int row = i * kT + 16 * wv + Mma<T>::row(lane, e);
-        if (col < n && row <= col) A[(int64_t)row * ld + col] = acc[c][e];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int col = j * kT + 16 * c + q;
+          if (col < n && row <= col) p[col] = acc[c][e];
+        }
+        if (e < 3) {
+          const int d = Mma<T>::row(0, e + 1) - Mma<T>::row(0, e);
+          row += d;
+          p += d * ld;
+        }
       }
     }
     return;
@@ -156,25 +208,35 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
   const int j = k + t;
   const int kb = min(kT, n - k0);
   const int ctiles = j > k ? 8 : 4;
-  if (k > 0) {
-    load_rows(A, ld, n, k0 - kT, k0, P, 0);
-    if (j > k) load_rows(A, ld, n, k0 - kT, j * kT, P, kT);
-  }
   {
+    T vk[kRowsPer], vj[kRowsPer];
+    if (k > 0) {
+      fetch_rows(A, ld, n, k0 - kT, k0, vk);
+      if (j > k) fetch_rows(A, ld, n, k0 - kT, j * kT, vj);
+    }
     M4 acc[8];
+    int row = min(k0 + 16 * wv + Mma<T>::row(lane, 0), n - 1);
+    const T* p = A + (int64_t)row * ld;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      if (c >= ctiles || (c < 4 && c < wv)) continue;  // uniform
-      const int cl = 16 * (c & 3) + q;
-      const int col = (c < 4 ? k0 : j * kT) + cl, cc = min(col, n - 1);
+    for (int e = 0; e < 4; ++e) {
+      const int r = 16 * wv + Mma<T>::row(lane, e);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int r = 16 * wv + Mma<T>::row(lane, e);
-        const T v = sign * A[(int64_t)min(k0 + r, cc) * ld + cc];
+      for (int c = 0; c < 8; ++c) {
+        if (c >= ctiles || (c < 4 && c < wv)) continue;  // uniform
+        const int cl = 16 * (c & 3) + q;
+        const int col = (c < 4 ? k0 : j * kT) + cl;
+        const T v = sign * p[min(col, n - 1)];
         const bool in = c < 4 ? (r <= cl && cl < kb) : col < n;
-        // past the last row the diagonal tile continues as the identity
+        // past the last row the diagonal tile continues as the identity;
+        // what lies below the diagonal is loaded and not used
         acc[c][e] = in ? v : (c < 4 && r == cl) ? T(1) : T(0);
       }
+      if (e < 3) step_rows(p, row, Mma<T>::row(0, e + 1) - Mma<T>::row(0, e), n, ld);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (k > 0) {
+      stash_rows(vk, n, k0, P, 0);
+      if (j > k) stash_rows(vj, n, j * kT, P, kT);
     }
     __syncthreads();
     if (k > 0) {
@@ -221,8 +283,13 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
         constexpr int p = decltype(T_)::value;
         const T d = from_lane(c[p], p);
         if (!(d > T(0)) && fail == 0) fail = k0 + r0 + p + 1;
-        const T u = sqrt(d);  // NaN for a negative pivot
-        const T inv = T(1) / u;
+        T u, inv;
+        if (root_range(d)) {  // uniform
+          pivot_root(d, u, inv);
+        } else {
+          u = sqrt(d);  // NaN for a negative pivot
+          inv = T(1) / u;
+        }
         c[p] = ln == p ? u : c[p] * inv;
         unroll<p + 1, kS>([&](auto I_) __attribute__((always_inline)) {
           constexpr int i = decltype(I_)::value;
@@ -265,39 +332,48 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
     // U_kj (all 64 rows exist), and zeros below the diagonal in tile (j, k);
     // row 0 of tile (k + 1, k) holds the diagonal of U_kk until the next launch
     const int col = j * kT + lane;
-    for (int r = wv; r < kT; r += 4) {
-      if (col < n) A[(int64_t)(k0 + r) * ld + col] = M[r * kLd + kT + lane];
-      const int zr = j * kT + r;
-      if (zr < n && !(j == k + 1 && r == 0)) A[(int64_t)zr * ld + k0 + lane] = T(0);
+    T* up = A + (int64_t)(k0 + wv) * ld + col;
+    T* lo = A + (int64_t)(j * kT + wv) * ld + k0 + lane;
+#pragma unroll 4
+    for (int r = wv; r < kT; r += 4, up += 4 * ld, lo += 4 * ld) {
+      if (col < n) *up = M[r * kLd + kT + lane];
+      if (j * kT + r < n && !(j == k + 1 && r == 0)) *lo = T(0);
     }
     return;
   }
   if (k > 0) {
-    // the diagonal tile of the launch before moves to its place
+    // the diagonal tile of the launch before moves to its place: row r of its
+    // strictly lower triangle holds column r of the factor above the diagonal
     const int p0 = k0 - kT;
-    for (int e = tid; e < kT * kT; e += kThreads) {
-      const int r = e / kT, c = e % kT;
-      if (r < c) P[r * kLd + c] = A[(int64_t)(p0 + c) * ld + p0 + r];
-      if (r == c) P[r * kLd + c] = A[(int64_t)k0 * ld + p0 + c];
-      if (r > c) P[r * kLd + c] = T(0);
+    T v[kRowsPer];
+    const T* p = A + (int64_t)(p0 + wv) * ld + p0 + lane;
+#pragma unroll
+    for (int u = 0; u < kRowsPer; ++u, p += 4 * ld) v[u] = *p;
+    const T dg = A[(int64_t)k0 * ld + p0 + lane];
+#pragma unroll
+    for (int u = 0; u < kRowsPer; ++u) {
+      const int r = wv + 4 * u;
+      if (lane < r) P[lane * kLd + r] = v[u];
+      if (lane > r) P[lane * kLd + r] = T(0);
+      if (lane == r) P[lane * kLd + r] = dg;
     }
     __syncthreads();  // every stored value is read before it is overwritten
-    for (int e = tid; e < kT * kT; e += kThreads) {
-      const int r = e / kT, c = e % kT;
-      A[(int64_t)(p0 + r) * ld + p0 + c] = P[r * kLd + c];
-    }
+    T* d = A + (int64_t)(p0 + wv) * ld + p0 + lane;
+#pragma unroll 4
+    for (int u = 0; u < kRowsPer; ++u, d += 4 * ld) *d = P[(wv + 4 * u) * kLd + lane];
     if (tid < kT) A[(int64_t)k0 * ld + p0 + tid] = T(0);
   }
   const bool last = k == nt - 1;
-  for (int e = tid; e < kT * kT; e += kThreads) {
-    const int r = e / kT, c = e % kT;
-    if (r >= kb || c >= kb) continue;
+  T* d = A + (int64_t)(k0 + wv) * ld + k0 + lane;
+#pragma unroll 4
+  for (int r = wv; r < kT; r += 4, d += 4 * ld) {
+    if (r >= kb || lane >= kb) continue;
     if (last) {
-      A[(int64_t)(k0 + r) * ld + k0 + c] = r <= c ? M[r * kLd + c] : T(0);
-    } else if (r > c) {
-      A[(int64_t)(k0 + r) * ld + k0 + c] = M[c * kLd + r];
-    } else if (r == c) {
-      A[(int64_t)(k0 + kT) * ld + k0 + c] = M[r * kLd + c];
+      *d = r <= lane ? M[r * kLd + lane] : T(0);
+    } else if (r > lane) {
+      *d = M[lane * kLd + r];
+    } else if (r == lane) {
+      A[(int64_t)(k0 + kT) * ld + k0 + lane] = M[r * kLd + lane];
     }
   }
   if (tid == 0 && (k == 0 || (fail && info[sys] == 0))) info[sys] = fail;
@@ -315,18 +391,19 @@ __global__ __launch_bounds__(kThreads) void chol_fail_kernel(int n, T* __restric
 }
 
 // ---------------------------------------------------------------------------
-// U^T U x = b, one right-hand side per system, one 1024-thread workgroup each.
-// Thread t holds columns t, t + 1024, ... of the vector in LDS and reads rows
-// of U (coalesced) in both directions:
+// U^T U x = b, one right-hand side per system, one 512-thread workgroup each.
+// The vector is in LDS; thread t takes every 512th column right of the block
+// at hand and reads rows of U (coalesced) in both directions:
 //   forward   y_j -= sum over the block's rows i of U_ij y_i, right-looking;
 //   backward  sum over columns j of U_ij x_j for the block's rows, left-looking,
 //             a wave reduce-scatter and a sum over waves in a fixed order.
-// The kRows x 1 values a thread needs for its first column of the next block
-// are loaded before the current block's chain of divisions starts, so that
-// the loads' latency is hidden by it.  That chain (kRows steps by one wave,
-// multipliers in registers) bounds the solve.
+// What a thread needs for its first two columns of the next block, and the next
+// but one diagonal block, are loaded one block ahead, and the barriers order
+// LDS only, so no block waits for memory.  The chain of R steps by one wave,
+// multipliers in registers, bounds the solve.
 // ---------------------------------------------------------------------------
-constexpr int kSolveThreads = 1024;
+constexpr int kSolveThreads = 512;
+constexpr int kSolveCols = 2;  // columns per thread that are loaded ahead
 constexpr int kSolveWaves = kSolveThreads / kWave;
 
 template <typename T>
@@ -346,7 +423,7 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
   __shared__ T rd[2][R];                  // reciprocals of their diagonals
   const T* U = u + (int64_t)blockIdx.x * u_stride;
   T* B = b + (int64_t)blockIdx.x * b_stride;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t ld = n;
   const int blocks = (n + R - 1) / R;
   // the vector: in LDS, or in place in global memory where it would not fit
@@ -366,46 +443,90 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
     for (int i = tid; i < blocks * R; i += kSolveThreads) ys[i] = i < n ? B[i] : T(0);
   }
 
-  // threads 0 .. R * R - 1 carry the diagonal block of block p through here
-  T dv = T(0);
-  const int di = tid / R, dj = tid % R;
+  // the diagonal block of block p passes through dv
+  constexpr int kDv = (R * R + kSolveThreads - 1) / kSolveThreads;
+  T dv[kDv] = {};
+  const int dj = tid % R;
   auto fetch_diag = [&](int p) {
-    if (tid < R * R) {
-      const int j = min(p * R + dj, n - 1);
-      dv = U[(int64_t)min(p * R + di, j) * ld + j];
+#pragma unroll
+    for (int h = 0; h < kDv; ++h) {
+      const int di = (tid + h * kSolveThreads) / R;
+      if (di < R) {
+        const int j = min(p * R + dj, n - 1);
+        dv[h] = U[(int64_t)min(p * R + di, j) * ld + j];
+      }
     }
   };
   auto stash_diag = [&](int p) {
-    if (tid < R * R) {
-      const bool in = p * R + dj < n && dj >= di;
-      D[p & 1][di][dj] = in ? dv : T(0);
-      if (di == dj) rd[p & 1][di] = in ? T(1) / dv : T(0);  // padding solves to 0
+#pragma unroll
+    for (int h = 0; h < kDv; ++h) {
+      const int di = (tid + h * kSolveThreads) / R;
+      if (di < R) {
+        const bool in = p * R + dj < n && dj >= di;
+        D[p & 1][di][dj] = in ? dv[h] : T(0);
+        if (di == dj) rd[p & 1][di] = in ? T(1) / dv[h] : T(0);  // padding solves to 0
+      }
     }
   };
   // column c, the R rows of block p (rows clamped; clamped ones meet y = 0)
-  T v[R];
-  auto fetch = [&](int p, int c) {
-    const int cc = min(c, n - 1);
+  T v[kSolveCols][R], nx[kSolveCols][R];
+  auto fetch = [&](int p, int c, T (&to)[R]) {
+    const int rows = n - p * R;  // rows that exist from the block's first one on
+    const unsigned cc = min(c, n - 1);
+    const T* at = U + (int64_t)(p * R) * ld;  // uniform: stepped on the scalar unit
 #pragma unroll
-    for (int i = 0; i < R; ++i) v[i] = U[(int64_t)min(p * R + i, n - 1) * ld + cc];
+    for (int i = 0; i < R; ++i) {
+      to[i] = at[cc];
+      at += i + 1 < rows ? ld : 0;
+    }
+  };
+  // the columns loaded ahead, of block p, from column c on
+  auto fetch_ahead = [&](int p, int c) {
+#pragma unroll
+    for (int h = 0; h < kSolveCols; ++h)
+      if (c + h * kSolveThreads < n) fetch(p, c + h * kSolveThreads + tid, nx[h]);  // uniform
+  };
+  auto take_ahead = [&]() {
+#pragma unroll
+    for (int h = 0; h < kSolveCols; ++h)
+#pragma unroll
+      for (int i = 0; i < R; ++i) v[h][i] = nx[h][i];
+  };
+#pragma unroll
+  for (int h = 0; h < kSolveCols; ++h)
+#pragma unroll
+    for (int i = 0; i < R; ++i) nx[h][i] = T(0);
+  // the vector in global memory needs the barrier that orders global memory
+  auto barrier = [&]() {
+    if constexpr (InLds) {
+      lds_barrier();
+    } else {
+      __syncthreads();
+    }
   };
 
   // ---- U^T y = b
   fetch_diag(0);
   stash_diag(0);
+  fetch_diag(min(1, blocks - 1));
+  fetch_ahead(0, R);
   __syncthreads();
   for (int p = 0; p < blocks; ++p) {
     const int c0 = p * R + R;
-    fetch(p, c0 + tid);
-    if (p + 1 < blocks) fetch_diag(p + 1);
+    take_ahead();
+    if (p + 1 < blocks) {
+      stash_diag(p + 1);
+      fetch_ahead(p + 1, c0 + R);
+      fetch_diag(min(p + 2, blocks - 1));
+    }
     if (wv == 0) {
-      T z = lane < R ? get(p * R + lane) : T(0);
-      int ln = lane;  // opaque per block: lane masks are not held across blocks
+      T z = get(p * R + lane % R);
+      int ln = lane % R;  // lanes past R repeat the others; opaque per block: lane masks are not held across blocks
       asm volatile("" : "+v"(ln));
-      const T r = lane < R ? rd[p & 1][lane] : T(0);
+      const T r = rd[p & 1][lane % R];
       T m[R];
 #pragma unroll
-      for (int i = 0; i < R; ++i) m[i] = lane < R ? D[p & 1][i][lane] : T(0);
+      for (int i = 0; i < R; ++i) m[i] = D[p & 1][i][lane % R];
 #pragma unroll
       for (int i = 0; i < R; ++i) {
         if (ln == i) z *= r;
@@ -414,45 +535,57 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
       }
       if (lane < R) put(p * R + lane, z);
     }
-    __syncthreads();
-    if (p + 1 < blocks) stash_diag(p + 1);
-    for (int c = c0 + tid; c < n; c += kSolveThreads) {
-      if (c >= c0 + kSolveThreads) fetch(p, c);
-      T s = T(0);
+    barrier();
+    if (c0 + (wv << 6) < n) {  // uniform
+      T yb[R];
 #pragma unroll
-      for (int i = 0; i < R; ++i) s += v[i] * get(p * R + i);
-      put(c, get(c) - s);
+      for (int i = 0; i < R; ++i) yb[i] = get(p * R + i);
+      auto push = [&](int c, const T (&e)[R]) {
+        T s = T(0);
+#pragma unroll
+        for (int i = 0; i < R; ++i) s += e[i] * yb[i];
+        if (c < n) put(c, get(c) - s);
+      };
+#pragma unroll
+      for (int h = 0; h < kSolveCols; ++h) push(c0 + h * kSolveThreads + tid, v[h]);
+      for (int c = c0 + kSolveCols * kSolveThreads + tid; c < n; c += kSolveThreads) {
+        fetch(p, c, v[0]);
+        push(c, v[0]);
+      }
     }
-    __syncthreads();
+    barrier();
   }
 
   // ---- U x = y
   fetch_diag(blocks - 1);
   stash_diag(blocks - 1);
+  fetch_diag(max(blocks - 2, 0));
+  fetch_ahead(max(blocks - 2, 0), (blocks - 1) * R);
   if (tid < kSolveWaves * R) part[tid / R][tid % R] = T(0);
   __syncthreads();
   for (int p = blocks - 1; p >= 0; --p) {
     // the products with the columns solved so far, except those of the block
     // solved last, are in part; this block's rows of those columns follow
     if (p > 0) {
-      fetch_diag(p - 1);
-      fetch(p - 1, p * R + tid);
+      take_ahead();
+      stash_diag(p - 1);
+      fetch_ahead(max(p - 2, 0), (p - 1) * R);
+      fetch_diag(max(p - 2, 0));
     }
     if (wv == 0) {
-      int ln = lane;
+      int ln = lane % R;
       asm volatile("" : "+v"(ln));
-      T z = T(0);
-      if (lane < R) {
-        z = get(p * R + lane);
+      T z = get(p * R + lane % R);
+      {
         T s = T(0);
 #pragma unroll
-        for (int w = 0; w < kSolveWaves; ++w) s += part[w][lane];
+        for (int w = 0; w < kSolveWaves; ++w) s += part[w][lane % R];
         z -= s;
       }
-      const T r = lane < R ? rd[p & 1][lane] : T(0);
+      const T r = rd[p & 1][lane % R];
       T m[R];
 #pragma unroll
-      for (int i = 0; i < R; ++i) m[i] = lane < R ? D[p & 1][lane][i] : T(0);
+      for (int i = 0; i < R; ++i) m[i] = D[p & 1][lane % R][i];
 #pragma unroll
       for (int i = R - 1; i >= 0; --i) {
         if (ln == i) z *= r;
@@ -461,18 +594,23 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
       }
       if (lane < R) put(p * R + lane, z);
     }
-    __syncthreads();
+    barrier();
     if (p > 0) {
-      stash_diag(p - 1);
       T s[R];
 #pragma unroll
       for (int i = 0; i < R; ++i) s[i] = T(0);
       const int c0 = p * R;
-      for (int c = c0 + tid; c < n; c += kSolveThreads) {
-        if (c >= c0 + kSolveThreads) fetch(p - 1, c);
-        const T x = get(c);
+      auto pull = [&](int c, const T (&e)[R]) {
+        const T x = c < n ? get(c) : T(0);
 #pragma unroll
-        for (int i = 0; i < R; ++i) s[i] += v[i] * x;
+        for (int i = 0; i < R; ++i) s[i] += e[i] * x;
+      };
+#pragma unroll
+      for (int h = 0; h < kSolveCols; ++h)
+        if (c0 + h * kSolveThreads < n) pull(c0 + h * kSolveThreads + tid, v[h]);
+      for (int c = c0 + kSolveCols * kSolveThreads + tid; c < n; c += kSolveThreads) {
+        fetch(p - 1, c, v[0]);
+        pull(c, v[0]);
       }
       if (c0 + wv * kWave < n || p == blocks - 1) {
         const T t = wave_reduce_scatter<R>(s, lane);
@@ -480,7 +618,7 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
         if ((lane & ((1 << kShift) - 1)) == 0) part[wv][lane >> kShift] = t;
       }
     }
-    __syncthreads();
+    barrier();
   }
   for (int i = tid; i < n; i += kSolveThreads) {
     const T x = get(i);
