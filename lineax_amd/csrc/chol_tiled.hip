@@ -129,7 +129,8 @@ __device__ __forceinline__ void step_rows(P& p, int& row, int steps, int n, int6
 }
 
 // Launch k of the factorisation; nt tiles per side.  Workgroups [0, batch *
-// (nt - k)) are the panel tiles, the rest the trailing tiles.
+// (nt - k)) are the panel tiles; the next batch of them moves the diagonal
+// tile of launch k - 1 into place; the rest are the trailing tiles.
 template <typename T>
 __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_kernel(int64_t batch, int n, int k, int nt, T* __restrict__ a,
                                                              int64_t a_stride, int negate,
@@ -149,9 +150,32 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
   // and launch 1 (all others)
   const T sign = (negate && k <= 1) ? T(-1) : T(1);
 
-  if (t >= nt - k) {
+  if (k > 0 && t == nt - k) {
+    // ---- the diagonal tile of the launch before moves to its place: row r of its
+    // strictly lower triangle holds column r of the factor above the diagonal
+    const int p0 = k0 - kT;
+    T v[kRowsPer];
+    const T* p = A + (int64_t)(p0 + wv) * ld + p0 + lane;
+#pragma unroll
+    for (int u = 0; u < kRowsPer; ++u, p += 4 * ld) v[u] = *p;
+    const T dg = A[(int64_t)k0 * ld + p0 + lane];
+#pragma unroll
+    for (int u = 0; u < kRowsPer; ++u) {
+      const int r = wv + 4 * u;
+      if (lane < r) P[lane * kLd + r] = v[u];
+      if (lane > r) P[lane * kLd + r] = T(0);
+      if (lane == r) P[lane * kLd + r] = dg;
+    }
+    __syncthreads();  // every stored value is read before it is overwritten
+    T* d = A + (int64_t)(p0 + wv) * ld + p0 + lane;
+#pragma unroll 4
+    for (int u = 0; u < kRowsPer; ++u, d += 4 * ld) *d = P[(wv + 4 * u) * kLd + lane];
+    if (tid < kT) A[(int64_t)k0 * ld + p0 + tid] = T(0);
+    return;
+  }
+  if (t > nt - k) {
     // ---- trailing tile (i, j), k < i <= j
-    t -= nt - k;
+    t -= nt - k + 1;
     int i = k + 1;
     while (t >= nt - i) {
       t -= nt - i;
@@ -185,6 +209,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
       for (int c = 0; c < 4; ++c) acc[c] = Mma<T>::mul(av, Ps[kT + 16 * c + q], acc[c]);
     }
     {
+      const bool whole = i < j && j + 1 < nt;  // uniform
       int row = i * kT + 16 * wv + Mma<T>::row(lane, 0);
       T* p = A + (int64_t)row * ld;
 #pragma unroll
@@ -192,7 +217,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const int col = j * kT + 16 * c + q;
-          if (col < n && row <= col) p[col] = acc[c][e];
+          if (whole || (col < n && row <= col)) p[col] = acc[c][e];
         }
         if (e < 3) {
           const int d = Mma<T>::row(0, e + 1) - Mma<T>::row(0, e);
@@ -208,55 +233,58 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
   const int j = k + t;
   const int kb = min(kT, n - k0);
   const int ctiles = j > k ? 8 : 4;
-  {
+  auto load_apply = [&](auto Tiles_) __attribute__((always_inline)) {
+    constexpr int kTiles = decltype(Tiles_)::value;  // 16-column tiles: 4, or 8 with tile (k, j)
     T vk[kRowsPer], vj[kRowsPer];
     if (k > 0) {
       fetch_rows(A, ld, n, k0 - kT, k0, vk);
-      if (j > k) fetch_rows(A, ld, n, k0 - kT, j * kT, vj);
+      if (kTiles == 8) fetch_rows(A, ld, n, k0 - kT, j * kT, vj);
     }
-    M4 acc[8];
+    M4 acc[kTiles];
     int row = min(k0 + 16 * wv + Mma<T>::row(lane, 0), n - 1);
     const T* p = A + (int64_t)row * ld;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int r = 16 * wv + Mma<T>::row(lane, e);
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        if (c >= ctiles || (c < 4 && c < wv)) continue;  // uniform
-        const int cl = 16 * (c & 3) + q;
-        const int col = (c < 4 ? k0 : j * kT) + cl;
-        const T v = sign * p[min(col, n - 1)];
-        const bool in = c < 4 ? (r <= cl && cl < kb) : col < n;
-        // past the last row the diagonal tile continues as the identity;
-        // what lies below the diagonal is loaded and not used
-        acc[c][e] = in ? v : (c < 4 && r == cl) ? T(1) : T(0);
-      }
+      for (int c = 0; c < kTiles; ++c) acc[c][e] = p[min((c < 4 ? k0 : j * kT) + 16 * (c & 3) + q, n - 1)];
       if (e < 3) step_rows(p, row, Mma<T>::row(0, e + 1) - Mma<T>::row(0, e), n, ld);
     }
     __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 16 * wv + Mma<T>::row(lane, e);
+#pragma unroll
+      for (int c = 0; c < kTiles; ++c) {
+        const int cl = 16 * (c & 3) + q;
+        const bool in = c < 4 ? (r <= cl && cl < kb) : j * kT + cl < n;
+        // past the last row the diagonal tile continues as the identity; what
+        // lies below the diagonal is not used (16 x 16 tiles there are
+        // carried along: leaving them out would split the loops by wave)
+        acc[c][e] = in ? sign * acc[c][e] : (c < 4 && r == cl) ? T(1) : T(0);
+      }
+    }
     if (k > 0) {
       stash_rows(vk, n, k0, P, 0);
-      if (j > k) stash_rows(vj, n, j * kT, P, kT);
-    }
-    __syncthreads();
-    if (k > 0) {
-#pragma unroll 2
+      if (kTiles == 8) stash_rows(vj, n, j * kT, P, kT);
+      __syncthreads();
+#pragma unroll 4
       for (int s = 0; s < kT; s += 4) {
         const T* Ps = P + (s + g) * kLd;
         const T av = -Ps[16 * wv + q];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          if (c >= ctiles || (c < 4 && c < wv)) continue;
-          acc[c] = Mma<T>::mul(av, Ps[16 * c + q], acc[c]);
-        }
+        for (int c = 0; c < kTiles; ++c) acc[c] = Mma<T>::mul(av, Ps[16 * c + q], acc[c]);
       }
     }
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      if (c >= ctiles || (c < 4 && c < wv)) continue;
+    for (int c = 0; c < kTiles; ++c) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) M[(16 * wv + Mma<T>::row(lane, e)) * kLd + 16 * c + q] = acc[c][e];
     }
+  };
+  if (j > k) {
+    load_apply(std::integral_constant<int, 8>{});
+  } else {
+    load_apply(std::integral_constant<int, 4>{});
   }
   __syncthreads();
 
@@ -340,28 +368,6 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
       if (j * kT + r < n && !(j == k + 1 && r == 0)) *lo = T(0);
     }
     return;
-  }
-  if (k > 0) {
-    // the diagonal tile of the launch before moves to its place: row r of its
-    // strictly lower triangle holds column r of the factor above the diagonal
-    const int p0 = k0 - kT;
-    T v[kRowsPer];
-    const T* p = A + (int64_t)(p0 + wv) * ld + p0 + lane;
-#pragma unroll
-    for (int u = 0; u < kRowsPer; ++u, p += 4 * ld) v[u] = *p;
-    const T dg = A[(int64_t)k0 * ld + p0 + lane];
-#pragma unroll
-    for (int u = 0; u < kRowsPer; ++u) {
-      const int r = wv + 4 * u;
-      if (lane < r) P[lane * kLd + r] = v[u];
-      if (lane > r) P[lane * kLd + r] = T(0);
-      if (lane == r) P[lane * kLd + r] = dg;
-    }
-    __syncthreads();  // every stored value is read before it is overwritten
-    T* d = A + (int64_t)(p0 + wv) * ld + p0 + lane;
-#pragma unroll 4
-    for (int u = 0; u < kRowsPer; ++u, d += 4 * ld) *d = P[(wv + 4 * u) * kLd + lane];
-    if (tid < kT) A[(int64_t)k0 * ld + p0 + tid] = T(0);
   }
   const bool last = k == nt - 1;
   T* d = A + (int64_t)(k0 + wv) * ld + k0 + lane;
@@ -633,14 +639,14 @@ int factor_t(hipStream_t st, int64_t batch, int n, T* a, int64_t stride, int neg
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (e != hipSuccess) return hip_error(e, "hipFuncSetAttribute(chol_tile_kernel)");
   const int nt = (n + kT - 1) / kT;
-  const int64_t most = (int64_t)nt + (int64_t)nt * (nt - 1) / 2;  // tiles of launch 1, the widest, or of launch 0
+  const int64_t most = (int64_t)nt + 1 + (int64_t)nt * (nt - 1) / 2;  // tiles of launch 1, the widest, or of launch 0
   // a grid holds fewer than 2^32 threads
   const int64_t chunk = std::max<int64_t>(1, (int64_t(1) << 23) / most);
   for (int64_t s0 = 0; s0 < batch; s0 += chunk) {
     const int64_t cnt = std::min(chunk, batch - s0);
     for (int k = 0; k < nt; ++k) {
       const int64_t rest = nt - k - 1;
-      const int64_t tiles = nt - k + (k > 0 ? rest * (rest + 1) / 2 : 0);
+      const int64_t tiles = nt - k + (k > 0 ? 1 + rest * (rest + 1) / 2 : 0);
       chol_tile_kernel<T><<<dim3((unsigned)(tiles * cnt)), kThreads, smem, st>>>(cnt, n, k, nt, a + s0 * stride, stride,
                                                                                   negate, info + s0);
     }
