@@ -3,13 +3,14 @@
 // Three tiers, chosen by order n:
 //  * n <= 64: one lane per row in registers, 64/LPS systems per wave; the
 //    scaled pivot row is broadcast through a double-buffered LDS row.
-//  * n <= 256 (float) / 181 (double): one 256-thread workgroup per system.
-//    Float factors run the register-tiled 16-column panel factorisation of
-//    chol_uneven.hip (chol_factor_regs_f32); double factors, and all solves,
-//    keep the upper triangle resident in LDS in row-packed form (131.6 KB
-//    at n = 256): right-looking factorisation, triangular solves by one
-//    wave with the vector in registers.
-//  * larger n: 64-column panels over all workgroups (chol_tiled.hip).
+//  * n <= 256, float factors: the register-tiled 16-column panel
+//    factorisation of chol_uneven.hip (chol_factor_regs_f32), one workgroup
+//    per system.
+//  * n <= 256 (float) / 181 (double) solves, and double factors of many small
+//    systems: one 256-thread workgroup per system with the upper triangle in
+//    LDS in row-packed form (131.6 KB at n = 256): right-looking
+//    factorisation, triangular solves by one wave with the vector in registers.
+//  * everything larger: 64-column panels over all workgroups (chol_tiled.hip).
 //
 // Failure semantics follow jax.scipy.linalg.cho_factor as lineax uses it
 // (lineax/_solver/cholesky.py:60): a non-positive or NaN pivot makes the
@@ -221,38 +222,68 @@ __device__ int lds_chol_factor(int n, T* L) {
 
 // Solves U^T U x = v in place, v distributed over one wave: lane l holds
 // v[l + 64 c].  Must be called by a whole wave with uniform control flow.
+// The chain of 2 n steps bounds it: the divisions are products with
+// reciprocals formed beforehand (one correction each), and the LDS reads of a
+// step are issued one step ahead.  256 double systems of order 150: 73 us
+// with a division and a waited LDS read per step.
 template <typename T>
 __device__ void wave_chol_solve(int n, const T* L, T (&v)[4]) {
   const int l = threadIdx.x & 63;
+  T d[4], rd[4];
+  bool plain = true;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int j = min(l + 64 * c, n - 1);
+    d[c] = L[packed_upper(n, j, j)];
+    rd[c] = T(1) / d[c];
+    plain = plain && plain_range(d[c]);
+  }
+  const bool fast = __all(plain);
+  auto over = [&](T x, int c) { return fast ? divide(x, d[c], rd[c]) : x / d[c]; };
   // U^T y = v, column oriented: y_k = v_k / U_kk, then v_j -= U_kj y_k.
+  auto row = [&](int k, T (&to)[4]) {
+    const int kc = min(k, n - 1);
+    const T* R = L + packed_upper(n, kc, kc) - kc;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) to[c] = R[max(min(l + 64 * c, n - 1), kc)];
+  };
+  T cur[4], nxt[4];
+  row(0, nxt);
 #pragma unroll
   for (int c0 = 0; c0 < 4; ++c0) {
     const int kend = min(64, n - 64 * c0);
     for (int kk = 0; kk < kend; ++kk) {
       const int k = 64 * c0 + kk;
-      const int rk = packed_upper(n, k, k);
-      const T yk = bcast_lane(v[c0], kk) / L[rk];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) cur[c] = nxt[c];
+      row(k + 1, nxt);
+      const T yk = bcast_lane(over(v[c0], c0), kk);
       if (l == kk) v[c0] = yk;
 #pragma unroll
-      for (int c = c0; c < 4; ++c) {
-        const int j = l + 64 * c;
-        if (j > k && j < n) v[c] -= L[rk + (j - k)] * yk;
-      }
+      for (int c = c0; c < 4; ++c)
+        if (l + 64 * c > k) v[c] -= cur[c] * yk;
     }
   }
   // U x = y, column oriented: x_k = y_k / U_kk, then y_i -= U_ik x_k.
+  auto column = [&](int k, T (&to)[4]) {
+    const int kc = max(k, 0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) to[c] = L[packed_upper(n, min(l + 64 * c, kc), kc)];
+  };
+  column(n - 1, nxt);
 #pragma unroll
   for (int c0 = 3; c0 >= 0; --c0) {
     const int kend = min(64, n - 64 * c0);
     for (int kk = kend - 1; kk >= 0; --kk) {
       const int k = 64 * c0 + kk;
-      const T xk = bcast_lane(v[c0], kk) / L[packed_upper(n, k, k)];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) cur[c] = nxt[c];
+      column(k - 1, nxt);
+      const T xk = bcast_lane(over(v[c0], c0), kk);
       if (l == kk) v[c0] = xk;
 #pragma unroll
-      for (int c = 0; c <= c0; ++c) {
-        const int i = l + 64 * c;
-        if (i < k) v[c] -= L[packed_upper(n, i, k)] * xk;
-      }
+      for (int c = 0; c <= c0; ++c)
+        if (l + 64 * c < k) v[c] -= cur[c] * xk;
     }
   }
 }
@@ -323,6 +354,13 @@ void launch_chol_solve_small(hipStream_t s, int64_t batch, int n, const T* u, in
                      n, u, us, b, bs, negate);
 }
 
+// Double factors stay with one workgroup and LDS per system only where the
+// systems are small and many enough to fill the chip several times over: 2000
+// systems of order 80 take 401 us a call this way and 476 us in tiles, of
+// order 100 580 us and 536 us; 512 of order 80 236 us and 224 us.
+constexpr int kLdsFactorMax = 96;
+constexpr int64_t kLdsFactorBatch = 512;
+
 template <typename T>
 int lds_max_n() {
   return sizeof(T) == 4 ? 256 : 181;  // packed triangle <= 131.6 KB
@@ -338,7 +376,7 @@ int chol_factor_t(hipStream_t s, int64_t batch, int64_t n64, T* a, int64_t strid
   else if (sizeof(T) == 4 && n <= 256) {
     // register-tiled 16-column panels (chol_uneven.hip)
     return chol_factor_regs_f32(s, batch, n, reinterpret_cast<float*>(a), stride, negate, info);
-  } else if (n <= lds_max_n<T>()) {
+  } else if (n <= kLdsFactorMax && batch > kLdsFactorBatch) {
     const size_t shmem = static_cast<size_t>(n) * (n + 1) / 2 * sizeof(T);
     if (int rc = allow_lds(chol_factor_lds_kernel<T>, shmem)) return rc;
     hipLaunchKernelGGL((chol_factor_lds_kernel<T>), dim3(static_cast<unsigned>(batch)), dim3(kWG), shmem, s, n, a,

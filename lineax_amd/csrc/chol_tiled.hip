@@ -1,6 +1,6 @@
-// Cholesky factorisation (potrf, upper: A = U^T U) of orders past the
-// one-workgroup tiers of chol.hip, in place, float32 and float64, and the
-// matching solve.
+// Cholesky factorisation (potrf, upper: A = U^T U) in 64-column panels over
+// all workgroups, in place, float32 and float64 (chol.hip says which calls
+// come here), and the solve of the orders past its LDS tier.
 //
 // Factor: one launch per 64-column panel, all systems of the batch and all
 // 64 x 64 tiles of the upper triangle at once.  Launch k
@@ -20,7 +20,9 @@
 // the launches.  A 16-row strip of a panel is therefore factored and solved
 // by the same instructions: lanes 0..15 of every wave hold the strip's
 // diagonal block, lanes 16..63 other columns, pivots and multipliers travel
-// by readlane and no barrier lies inside a strip.
+// by readlane and no barrier lies inside a strip.  One system of order 1000:
+// 17.6 us (float) and 25 us (double) a launch; one workgroup in global memory,
+// which this replaces, took 280 ms for the float one.
 //
 // Reference: lineax/_solver/cholesky.py:43-78 (cho_factor / cho_solve).
 #include <algorithm>
@@ -132,13 +134,16 @@ __device__ __forceinline__ void step_rows(P& p, int& row, int steps, int n, int6
 // (nt - k)) are the panel tiles; the next batch of them moves the diagonal
 // tile of launch k - 1 into place; the rest are the trailing tiles.
 template <typename T>
-__global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_kernel(int64_t batch, int n, int k, int nt, T* __restrict__ a,
+__global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 2) void chol_tile_kernel(int64_t batch, int n, int k, int nt, T* __restrict__ a,
                                                              int64_t a_stride, int negate,
                                                              int32_t* __restrict__ info) {
   using M4 = typename Mma<T>::acc;
   extern __shared__ __align__(16) unsigned char lxa_smem[];
-  T* P = reinterpret_cast<T*>(lxa_smem);  // [64][kLd]: rows of panel k - 1
-  T* M = P + kT * kLd;                    // [64][kLd]: diagonal tile and tile (k, j)
+  // [64][kLd]: P, rows of panel k - 1; then M, the diagonal tile and tile (k, j)
+  // (sharing the space lets two double workgroups onto a CU: 256 systems of
+  // order 150 take 34 us a launch instead of 48)
+  T* P = reinterpret_cast<T*>(lxa_smem);
+  T* M = P;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q = lane & 15, g = lane >> 4;
   const int64_t sys = blockIdx.x % batch;
@@ -274,6 +279,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 2 : 1) void chol_tile_ke
 #pragma unroll
         for (int c = 0; c < kTiles; ++c) acc[c] = Mma<T>::mul(av, Ps[16 * c + q], acc[c]);
       }
+      __syncthreads();  // P is M from here on
     }
 #pragma unroll
     for (int c = 0; c < kTiles; ++c) {
@@ -634,7 +640,7 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
 
 template <typename T>
 int factor_t(hipStream_t st, int64_t batch, int n, T* a, int64_t stride, int negate, int32_t* info) {
-  const size_t smem = sizeof(T) * 2 * kT * kLd;
+  const size_t smem = sizeof(T) * kT * kLd;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&chol_tile_kernel<T>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (e != hipSuccess) return hip_error(e, "hipFuncSetAttribute(chol_tile_kernel)");

@@ -93,17 +93,6 @@ __device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
   return v;
 }
 
-// Divisors for which x / d is x * (1 / d) and one correction: reciprocal and
-// residual stay normal.
-__device__ __forceinline__ bool plain_range(float d) { return fabsf(d) >= 0x1p-100f && fabsf(d) <= 0x1p100f; }
-__device__ __forceinline__ bool plain_range(double d) { return fabs(d) >= 0x1p-900 && fabs(d) <= 0x1p900; }
-
-template <typename T>
-__device__ __forceinline__ T divide(T x, T d, T rd) {
-  const T q = x * rd;
-  return fma(fma(-d, q, x), rd, q);
-}
-
 // S row slots per lane of the panel wave; InLds: the matrix is in LDS.
 template <typename T, int S, bool InLds>
 __global__ __launch_bounds__(kThreads) void lu_mid_factor_kernel(int n, T* __restrict__ a, int64_t a_stride,

@@ -163,6 +163,17 @@ __device__ __forceinline__ R wave_reduce_scatter(R (&v)[K], int lane) {
   return x;
 }
 
+// Divisors for which x / d is x * (1 / d) and one correction: reciprocal and
+// residual stay normal.
+__device__ __forceinline__ bool plain_range(float d) { return fabsf(d) >= 0x1p-100f && fabsf(d) <= 0x1p100f; }
+__device__ __forceinline__ bool plain_range(double d) { return fabs(d) >= 0x1p-900 && fabs(d) <= 0x1p900; }
+
+template <typename T>
+__device__ __forceinline__ T divide(T x, T d, T rd) {
+  const T q = x * rd;
+  return fma(fma(-d, q, x), rd, q);
+}
+
 // Index of element (i, j), j >= i, in a row-packed upper triangle of order n.
 __device__ __forceinline__ int packed_upper(int n, int i, int j) {
   return i * n - ((i * (i - 1)) >> 1) + (j - i);
