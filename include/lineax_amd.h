@@ -604,9 +604,10 @@ typedef struct {
   int32_t m, n, lda, ldb;
 } lxa_qr_desc; /* 56 bytes */
 
-/* Panel width of the blocked factorisation: 16 for float32, 8 for float64. */
+/* Panel width of the blocked factorisation (16 for both types). */
 int lxa_qr_block(int dtype);
-/* Scratch elements one system of order m x n needs in lxa_qr_factor. */
+/* Scratch elements one system of order m x n needs in lxa_qr_factor
+ * (one: the kernels use none, but work may not be NULL). */
 int lxa_qr_work_elems(int dtype, int64_t m, int64_t n, int64_t* elems);
 /* geqrf of every system (qr.py:62).  max_m / max_n / max_k bound m, n and
  * min(m, n) over the batch (they size the launch grids). */

@@ -1,33 +1,29 @@
 // Householder QR over uneven batches (geqrf / ormqr) and triangular solves
 // for gfx950.
 //
-// Factorisation (lxa_qr_factor) is blocked, right-looking, compact WY:
-// each panel step factors nb columns of every system and then updates the
-// systems' trailing columns:
-//
-//   panel   one 512-thread workgroup per system.  The panel (rows k..m-1,
-//           nb columns) lives in registers, up to eight rows x nb columns
-//           per thread, i.e. 4096 rows (a global-memory variant covers
-//           taller panels).  Per column one block reduction carries the
-//           norm below the diagonal (larfg) and the raw products of that
-//           column with the other panel columns, from which v^T A (larf)
-//           and v_a^T v_j (for the T factor) follow.
-//           The workgroup ends by forming T (larft) and writing tau, T and
-//           the panel back.
-//   trail   C <- (I - V T V^T)^T C = C - V (T^T (V^T C)) on the columns
-//           right of the panel: (1) partial V^T C per 256-row chunk and
-//           64-column block, (2) the chunk sum and T^T, (3) C -= V W.  Each
-//           pass is a coalesced sweep over C (read, read, read+write).
-//
-// Block sums are deterministic: a wave reduce-scatter (log2 K halving
-// exchanges, then a full reduction of one value per lane), then a fixed
-// order over waves.
+// Factorisation (lxa_qr_factor) is blocked, right-looking, compact WY, 16
+// columns at a time, one launch per panel (qr_step_kernel).  A 512-thread
+// workgroup owns 16 columns of one system and all their rows, in registers in
+// the layout of the matrix cores' results:
+//   update  C <- (I - V T V^T)^T C: W = V^T C, T^T W and C - V (T^T W) are
+//           matrix-core products whose inner index is permuted so that a
+//           result register is an operand register of the next product; C is
+//           read and written once per panel.
+//   panel   the workgroup that updated the columns next to the panel factors
+//           them at once, while the others are still updating theirs.  Lane
+//           q of each 16-lane row holds column q, so the products of column j
+//           with all others are one multiply-add per element (column j by a
+//           DPP row broadcast), the sum over a wave is two exchanges, and one
+//           barrier per column carries products, norm and diagonal row.
+// Panels taller than 4096 rows are factored from global memory by
+// qr_panel_kernel and updated in two sweeps over C.
 //
 // Reference: lineax/_solver/qr.py:55-92 calls jnp.linalg.qr(mode="raw")
 // (geqrf), jax.lax.linalg.ormqr and jax.scipy.linalg.solve_triangular; the
 // reflector convention here is LAPACK's (larfg: beta = -sign(alpha) ||x||,
 // tau = (beta - alpha) / beta, v = x / (alpha - beta), tau = 0 when x = 0).
 
+#include <algorithm>
 #include <type_traits>
 
 #include "lxa_common.h"
@@ -36,24 +32,15 @@ namespace lxa {
 namespace {
 
 template <typename T>
-struct QrCfg;
-template <>
-struct QrCfg<float> {
+struct QrCfg {
   static constexpr int NB = 16;
-};
-template <>
-struct QrCfg<double> {
-  static constexpr int NB = 8;
 };
 
 constexpr int kPanelThreads = 512;   // 2 waves per SIMD: 256 VGPRs each
 constexpr int kPanelWaves = kPanelThreads / kWave;
-constexpr int kPanelMaxRpt = 8;      // register panel: rows <= 4096
+constexpr int kStepMaxRows = 4096;   // tallest panel the step kernel factors
 constexpr int kBigThreads = 1024;    // apply / triangular solve workgroups
 constexpr int kBigWaves = kBigThreads / kWave;
-constexpr int kTrailCols = 64;
-constexpr int kTrailRows = 256;
-constexpr int kTrailThreads = 256;
 
 // Block sum of K values per thread over a workgroup of WAVES waves.
 // stage: LDS [WAVES][K]; out: LDS [K].  Every thread gets the sums.
@@ -124,10 +111,9 @@ __device__ __forceinline__ T vpick(int row, int diag, T stored) {
 }
 
 // ---------------------------------------------------------------------------
-// Panel factorisation.  RPT > 0: rows in registers (RPT per thread);
-// RPT == 0: rows in global memory (any height, slower).
+// Panel factorisation with the rows in global memory (any height).
 // ---------------------------------------------------------------------------
-template <typename T, int RPT>
+template <typename T>
 __global__ __launch_bounds__(kPanelThreads) void qr_panel_kernel(const lxa_qr_desc* __restrict__ descs, int k_all,
                                                                  const int32_t* __restrict__ kcol,
                                                                  T* __restrict__ a, T* __restrict__ tau,
@@ -139,7 +125,6 @@ __global__ __launch_bounds__(kPanelThreads) void qr_panel_kernel(const lxa_qr_de
   __shared__ T s_stage[kPanelWaves * KW];
   __shared__ T s_out[KW];
   __shared__ T s_diag[2][NB];  // the diagonal row of the current column
-  __shared__ T s_rows[RPT > 0 ? kPanelThreads : 1][NB + 1];  // staging of 512 panel rows
   __shared__ T s_g[NB][NB];    // s_g[a][j] = v_a^T v_j, a < j
 
   const lxa_qr_desc d = descs[blockIdx.x];
@@ -150,47 +135,8 @@ __global__ __launch_bounds__(kPanelThreads) void qr_panel_kernel(const lxa_qr_de
   const int nb = min(NB, kmax - k);
   const int tid = threadIdx.x;
   T* A = a + d.a_offset;
-  const int nr = RPT ? RPT : (m - k + kPanelThreads - 1) / kPanelThreads;
-
-  T regs[RPT ? RPT : 1][NB];
-  auto P = [&](int r, int c) -> T& {
-    if constexpr (RPT > 0) {
-      return regs[r][c];
-    } else {
-      return A[(int64_t)(k + tid + r * kPanelThreads) * lda + k + c];
-    }
-  };
-
-  if constexpr (RPT > 0) {
-    // rows k + r * 512 + [0, 512) pass through LDS: NB consecutive lanes read
-    // one row's NB contiguous entries, then each thread takes its own row
-#pragma unroll
-    for (int r = 0; r < RPT; ++r) {
-      const int base = k + r * kPanelThreads;
-      if (base < m) {  // uniform
-        // all NB loads in flight before any LDS write
-        T v[NB];
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-          const int e = tid + kPanelThreads * u, rr = e / NB, c = e % NB;
-          const int row = base + rr;
-          v[u] = (row < m && c < nb) ? A[(int64_t)row * lda + k + c] : T(0);
-        }
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-          const int e = tid + kPanelThreads * u;
-          s_rows[e / NB][e % NB] = v[u];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int c = 0; c < NB; ++c) regs[r][c] = s_rows[tid][c];
-        __syncthreads();
-      } else {
-#pragma unroll
-        for (int c = 0; c < NB; ++c) regs[r][c] = T(0);
-      }
-    }
-  }
+  const int nr = (m - k + kPanelThreads - 1) / kPanelThreads;
+  auto P = [&](int r, int c) -> T& { return A[(int64_t)(k + tid + r * kPanelThreads) * lda + k + c]; };
 
   T taus[NB];
   // the column loop at compile time (every register index a constant)
@@ -211,7 +157,6 @@ __global__ __launch_bounds__(kPanelThreads) void qr_panel_kernel(const lxa_qr_de
     T dots[KW];
 #pragma unroll
     for (int c = 0; c < KW; ++c) dots[c] = T(0);
-#pragma unroll
     for (int r = 0; r < nr; ++r) {
       const int row = k + tid + r * kPanelThreads;
       if (row < m && row > diag) {
@@ -246,7 +191,6 @@ __global__ __launch_bounds__(kPanelThreads) void qr_panel_kernel(const lxa_qr_de
     }
     // ---- scale x into v, put beta on the diagonal, and apply
     // (I - tau v v^T) to the panel columns right of j
-#pragma unroll
     for (int r = 0; r < nr; ++r) {
       const int row = k + tid + r * kPanelThreads;
       if (row < m && row >= diag) {
@@ -295,307 +239,365 @@ __global__ __launch_bounds__(kPanelThreads) void qr_panel_kernel(const lxa_qr_de
     for (int i = 0; i < NB; ++i)
       if (i == ra && i < nb) tau[d.tau_offset + k + i] = taus[i];
   }
-
-  if constexpr (RPT > 0) {
-    // the panel back through LDS, in the same coalesced order as the load
-#pragma unroll
-    for (int r = 0; r < RPT; ++r) {
-      const int base = k + r * kPanelThreads;
-      if (base < m) {  // uniform
-        __syncthreads();  // the previous chunk's readers are done
-#pragma unroll
-        for (int c = 0; c < NB; ++c) s_rows[tid][c] = regs[r][c];
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-          const int e = tid + kPanelThreads * u, rr = e / NB, c = e % NB;
-          const int row = base + rr;
-          if (row < m && c < nb) A[(int64_t)row * lda + k + c] = s_rows[rr][c];
-        }
-      }
-    }
-  }
 }
 
-// Loads the Householder vectors of rows [r0, r0 + kTrailRows) of the panel at
-// column k into LDS (with the implied unit diagonal and zeros above).
-template <typename T, int NB>
-__device__ __forceinline__ void load_v_chunk(T (*sv)[NB], const T* A, int lda, int m, int k, int nb, int r0,
-                                             int tid) {
-  // NB consecutive lanes read one row's NB entries (contiguous in memory)
-  static_assert(kTrailThreads % NB == 0 && kTrailRows % (kTrailThreads / NB) == 0, "tile shape");
-  const int j = tid % NB;
-  const int diag = k + j;
-  constexpr int kPer = kTrailRows / (kTrailThreads / NB);
-#pragma unroll
-  for (int t = 0; t < kPer; ++t) {
-    const int i = tid / NB + t * (kTrailThreads / NB);
-    const int row = r0 + i;
-    T v = T(0);
-    if (row < m && j < nb) v = row > diag ? A[(int64_t)row * lda + k + j] : (row == diag ? T(1) : T(0));
-    sv[i][j] = v;
-  }
-}
+// ---------------------------------------------------------------------------
+// One panel step for 16 columns of one system per workgroup.
+// ---------------------------------------------------------------------------
 
-// Rows of a trailing chunk handled per wave between waits: each wave issues
-// this many independent loads of C before using any of them.
-constexpr int kTrailBatch = 8;
-
-// (1) partial W = V^T C over one 256-row chunk and one 64-column block.
+// One 16 x 16 x 4 matrix-core product.  Lane l = 16 g + q: A operand
+// [q][inner g], B operand [inner g][q], result register e holds row row(g, e)
+// and column q.  Where the inner index of a product is the row index of an
+// earlier result, step e takes inner indices row(0..3, e), so that register e
+// of that result is the B operand as it stands.
 template <typename T>
-__global__ __launch_bounds__(kTrailThreads) void qr_trail_partial_kernel(const lxa_qr_desc* __restrict__ descs,
-                                                                        int k_all, const int32_t* __restrict__ kcol,
-                                                                        const T* __restrict__ a, T* __restrict__ work) {
+struct QrMma;
+template <>
+struct QrMma<float> {
+  typedef float acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mul(float a, float b, acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ constexpr int row(int g, int e) { return 4 * g + e; }
+};
+template <>
+struct QrMma<double> {
+  typedef double acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mul(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ constexpr int row(int g, int e) { return g + 4 * e; }
+};
+
+// The value of lane J of this lane's row of 16 (DPP row_newbcast; every lane
+// must be active).
+template <int J>
+__device__ __forceinline__ float row_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + J, 0xF, 0xF, false));
+}
+template <int J>
+__device__ __forceinline__ double row_bcast(double v) {
+  const uint64_t u = static_cast<uint64_t>(__double_as_longlong(v));
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0u, static_cast<uint32_t>(u), 0x150 + J, 0xF, 0xF, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0u, static_cast<uint32_t>(u >> 32), 0x150 + J, 0xF, 0xF, false);
+  return __longlong_as_double(static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo));
+}
+
+// What a launch does with the panel at column k.
+enum : int {
+  kStepPanel = 0,      // factor it (one workgroup per system)
+  kStepUpdate = 1,     // apply it to the columns on its right
+  kStepLookahead = 2,  // apply it, and factor the panel after it
+};
+
+// KR: 16-row tiles per wave held in registers (slot s of wave w is tile
+// w + 8 s of the rows from k on); KL: further ones in LDS (the register file
+// holds 2048 double or 3072 float rows beside what the products need).  KR = 0: any height, C read again for the update; no panel.
+template <typename T, int KR, int KL>
+__global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_desc* __restrict__ descs, int64_t count,
+                                                                int mode, int k_all,
+                                                                const int32_t* __restrict__ kcol, T* __restrict__ a,
+                                                                T* __restrict__ tau, T* __restrict__ tblk) {
   constexpr int NB = QrCfg<T>::NB;
-  __shared__ T sv[kTrailRows][NB];
-  __shared__ T sp[kTrailThreads / kWave][NB][kWave];
-  const lxa_qr_desc d = descs[blockIdx.z];
+  static_assert(NB == 16 && KR % 4 == 0, "16-column panels; slots go in groups of four");
+  constexpr int kWaves = kPanelWaves, kSpan = 16 * kWaves;  // rows per slot over the waves
+  using M4 = typename QrMma<T>::acc;
+  extern __shared__ __align__(16) unsigned char step_smem[];
+  T* far_slots = reinterpret_cast<T*>(step_smem);  // [KL][4][kPanelThreads]
+  __shared__ T s_w[kWaves][NB][NB + 1];
+  __shared__ T s_part[2][kWaves][NB];
+  __shared__ double s_norm[2][kWaves];
+  __shared__ T s_diag[2][NB];
+  __shared__ T s_g[NB][NB];  // s_g[c][j] = v_c^T v_j, c < j
+  __shared__ T s_tau[NB];
+
+  const int64_t sys = blockIdx.x % count;
+  const int blk = (int)(blockIdx.x / count);
+  const lxa_qr_desc d = descs[sys];
   const int m = d.m, n = d.n, lda = d.lda;
   const int kmax = min(m, n);
-  const int k = kcol ? kcol[blockIdx.z] : k_all;
+  const int k = kcol ? kcol[sys] : k_all;
   if (k >= kmax) return;
   const int nb = min(NB, kmax - k);
-  const int c0 = k + nb + kTrailCols * (int)blockIdx.x;
-  const int r0 = k + kTrailRows * (int)blockIdx.y;
-  if (c0 >= n || r0 >= m) return;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid >> 6;
-  const T* A = a + d.a_offset;
-  load_v_chunk<T, NB>(sv, A, lda, m, k, nb, r0, tid);
-  __syncthreads();
-  const int col = c0 + lane;
-  const bool cv = col < n;
-  T acc[NB];
-#pragma unroll
-  for (int j = 0; j < NB; ++j) acc[j] = T(0);
-  const int rows = min(kTrailRows, m - r0);
-  constexpr int kStep = kTrailThreads / kWave;
-  for (int i0 = wv; i0 < rows; i0 += kTrailBatch * kStep) {
-    T cb[kTrailBatch];
-#pragma unroll
-    for (int u = 0; u < kTrailBatch; ++u) {
-      const int i = i0 + u * kStep;
-      cb[u] = (cv && i < rows) ? A[(int64_t)(r0 + i) * lda + col] : T(0);
-    }
-    // rows in the same order as one at a time: the sums are unchanged
-#pragma unroll
-    for (int u = 0; u < kTrailBatch; ++u) {
-      const int i = i0 + u * kStep;
-      if (i < rows) {
-#pragma unroll
-        for (int j = 0; j < NB; ++j) acc[j] += sv[i][j] * cb[u];
-      }
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < NB; ++j) sp[wv][j][lane] = acc[j];
-  __syncthreads();
-  T* W = work + d.w_offset + (int64_t)blockIdx.y * NB * n;
-  for (int idx = tid; idx < NB * kWave; idx += kTrailThreads) {
-    const int j = idx >> 6, l = idx & (kWave - 1);
-    T s = T(0);
-#pragma unroll
-    for (int w = 0; w < kTrailThreads / kWave; ++w) s += sp[w][j][l];
-    if (c0 + l < n) W[(int64_t)j * n + c0 + l] = s;
-  }
-}
-
-// (2) W = sum over chunks, then W <- T^T W; stored in chunk slot 0.
-template <typename T>
-__global__ __launch_bounds__(kTrailThreads) void qr_trail_reduce_kernel(const lxa_qr_desc* __restrict__ descs,
-                                                                       int k_all, const int32_t* __restrict__ kcol,
-                                                                       const T* __restrict__ tblk,
-                                                                       T* __restrict__ work) {
-  constexpr int NB = QrCfg<T>::NB;
-  __shared__ T sw[NB][kWave];
-  __shared__ T st[NB][NB];
-  const lxa_qr_desc d = descs[blockIdx.y];
-  const int m = d.m, n = d.n;
-  const int kmax = min(m, n);
-  const int k = kcol ? kcol[blockIdx.y] : k_all;
-  if (k >= kmax) return;
-  const int nb = min(NB, kmax - k);
-  const int c0 = k + nb + kTrailCols * (int)blockIdx.x;
+  const int c0 = mode == kStepPanel ? k : k + nb + NB * blk;
   if (c0 >= n) return;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), g = tid >> 6;
-  const int chunks = (m - k + kTrailRows - 1) / kTrailRows;
-  T* W = work + d.w_offset;
-  const T* Tp = tblk + d.t_offset + (int64_t)(k / NB) * NB * NB;
-  if (tid < NB * NB) st[tid / NB][tid % NB] = Tp[tid];
-  const int col = c0 + lane;
-  for (int j = g; j < NB; j += kTrailThreads / kWave) {
-    T s = T(0);
-    if (col < n)
-      for (int ch = 0; ch < chunks; ++ch) s += W[((int64_t)ch * NB + j) * n + col];
-    sw[j][lane] = s;
-  }
-  __syncthreads();
-  for (int j = g; j < NB; j += kTrailThreads / kWave) {
-    T s = T(0);
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-      if (i <= j) s += st[i][j] * sw[i][lane];
-    if (col < n) W[(int64_t)j * n + col] = s;
-  }
-}
-
-// (3) C -= V W over one chunk and column block.
-template <typename T>
-__global__ __launch_bounds__(kTrailThreads) void qr_trail_update_kernel(const lxa_qr_desc* __restrict__ descs,
-                                                                       int k_all, const int32_t* __restrict__ kcol,
-                                                                       T* __restrict__ a,
-                                                                       const T* __restrict__ work) {
-  constexpr int NB = QrCfg<T>::NB;
-  __shared__ T sv[kTrailRows][NB];
-  const lxa_qr_desc d = descs[blockIdx.z];
-  const int m = d.m, n = d.n, lda = d.lda;
-  const int kmax = min(m, n);
-  const int k = kcol ? kcol[blockIdx.z] : k_all;
-  if (k >= kmax) return;
-  const int nb = min(NB, kmax - k);
-  const int c0 = k + nb + kTrailCols * (int)blockIdx.x;
-  const int r0 = k + kTrailRows * (int)blockIdx.y;
-  if (c0 >= n || r0 >= m) return;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q = lane & 15, g = lane >> 4;
   T* A = a + d.a_offset;
-  load_v_chunk<T, NB>(sv, A, lda, m, k, nb, r0, tid);
-  const int col = c0 + lane;
+  const int col = c0 + q;
   const bool cv = col < n;
-  const T* W = work + d.w_offset;
-  T w[NB];
+  const int rows = m - k;                                    // this step's rows
+  const int ns = max(0, ((rows + 15) / 16 - wv + kWaves - 1) / kWaves);  // this wave's tiles
+
+  // lane offsets of the four rows of a tile, from the row (k + kSpan * s)
+  int rel[4];
+  int64_t off[4];
 #pragma unroll
-  for (int j = 0; j < NB; ++j) w[j] = cv ? W[(int64_t)j * n + col] : T(0);
-  __syncthreads();
-  if (!cv) return;
-  const int rows = min(kTrailRows, m - r0);
-  constexpr int kStep = kTrailThreads / kWave;
-  for (int i0 = wv; i0 < rows; i0 += kTrailBatch * kStep) {
-    T cb[kTrailBatch];
+  for (int e = 0; e < 4; ++e) {
+    rel[e] = 16 * wv + QrMma<T>::row(g, e);
+    off[e] = (int64_t)rel[e] * lda;
+  }
+  auto base = [&](int s) { return A + (int64_t)min(k + kSpan * s, m - 1) * lda; };  // uniform
+  auto exists = [&](int s, int e) { return kSpan * s + rel[e] < rows; };
+  auto load = [&](int s) {
+    const T* p = base(s) + min(col, n - 1);
+    M4 v;
 #pragma unroll
-    for (int u = 0; u < kTrailBatch; ++u) {
-      const int i = i0 + u * kStep;
-      cb[u] = i < rows ? A[(int64_t)(r0 + i) * lda + col] : T(0);
+    for (int e = 0; e < 4; ++e) v[e] = p[exists(s, e) ? off[e] : 0];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = cv && exists(s, e) ? v[e] : T(0);
+    return v;
+  };
+  auto store = [&](int s, const M4& v) {
+    T* p = base(s) + col;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (cv && exists(s, e)) p[off[e]] = v[e];
+  };
+  // f(slot, value) over this wave's tiles
+  M4 acc[KR > 0 ? KR : 1];
+  auto each = [&](auto&& f) __attribute__((always_inline)) {
+    static_for<0, KR / 4>([&](auto G_) __attribute__((always_inline)) {
+      constexpr int s4 = 4 * decltype(G_)::value;
+      if (s4 < ns) {  // uniform; slots past the rows hold zeros
+#pragma unroll
+        for (int u = 0; u < 4; ++u) f(s4 + u, acc[s4 + u]);
+      }
+    });
+    for (int s = KR; s < (KL > 0 ? ns : 0); ++s) {
+      T* far = far_slots + (int64_t)(s - KR) * 4 * kPanelThreads + tid;
+      M4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = far[e * kPanelThreads];
+      f(s, v);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) far[e * kPanelThreads] = v[e];
+    }
+  };
+  if constexpr (KR > 0) each([&](int s, M4& v) __attribute__((always_inline)) { v = load(s); });
+
+  if (mode != kStepPanel) {
+    // ---- W = V^T C
+    const T* Tp = tblk + d.t_offset + (int64_t)(k / NB) * NB * NB;
+    T tt[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tt[e] = Tp[QrMma<T>::row(g, e) * NB + q];
+    const int vc = k + min(q, nb - 1);
+    auto project = [&](int s, const M4& c, M4 w) {
+      const T* p = base(s) + vc;
+      T v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = p[exists(s, e) ? off[e] : 0];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const T x = vpick(kSpan * s + rel[e], q, v[e]);
+        w = QrMma<T>::mul(exists(s, e) && q < nb ? x : T(0), c[e], w);
+      }
+      return w;
+    };
+    M4 w = {T(0), T(0), T(0), T(0)};
+    if constexpr (KR > 0) {
+      each([&](int s, M4& v) __attribute__((always_inline)) { w = project(s, v, w); });
+    } else {
+#pragma unroll 4
+      for (int s = 0; s < ns; ++s) w = project(s, load(s), w);
     }
 #pragma unroll
-    for (int u = 0; u < kTrailBatch; ++u) {
-      const int i = i0 + u * kStep;
-      if (i < rows) {
-        T s = T(0);
+    for (int e = 0; e < 4; ++e) s_w[wv][QrMma<T>::row(g, e)][q] = w[e];
+    __syncthreads();
 #pragma unroll
-        for (int j = 0; j < NB; ++j) s += sv[i][j] * w[j];
-        A[(int64_t)(r0 + i) * lda + col] = cb[u] - s;
+    for (int e = 0; e < 4; ++e) {
+      T x = T(0);
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) x += s_w[i][QrMma<T>::row(g, e)][q];
+      w[e] = x;
+    }
+    // ---- T^T W, then C - V (T^T W)
+    M4 tw = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tw = QrMma<T>::mul(tt[e], w[e], tw);
+    const int rq = 16 * wv + q;  // V by rows: row q of the tile
+    const int64_t offq = (int64_t)rq * lda;
+    auto subtract = [&](int s, M4 c) {
+      const bool in = kSpan * s + rq < rows;
+      const T* p = base(s) + (in ? offq : 0) + k;
+      T v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = p[min(QrMma<T>::row(g, e), nb - 1)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int j = QrMma<T>::row(g, e);
+        const T x = vpick(kSpan * s + rq, j, v[e]);
+        c = QrMma<T>::mul(in && j < nb ? -x : T(0), tw[e], c);
       }
+      return c;
+    };
+    if constexpr (KR > 0) {
+      each([&](int s, M4& v) __attribute__((always_inline)) { v = subtract(s, v); });
+    } else {
+#pragma unroll 4
+      for (int s = 0; s < ns; ++s) store(s, subtract(s, load(s)));
+    }
+  }
+  if constexpr (KR > 0) {
+    const int kn = mode == kStepPanel ? k : k + NB;  // the panel to factor
+    if (mode == kStepUpdate || blk != 0 || kn >= kmax) {
+      each([&](int s, M4& v) __attribute__((always_inline)) { store(s, v); });
+      return;
+    }
+    const int nbn = min(NB, kmax - kn);
+    const int t0 = (kn - k) / 16;  // tile with the panel's diagonal: slot 0 of wave t0
+    T sc = T(1);                   // scaling of this lane's column below its diagonal, applied when stored
+    static_for<0, NB>([&](auto J_) __attribute__((always_inline)) {
+      constexpr int j = decltype(J_)::value;
+      if (j >= nbn) return;  // uniform
+      constexpr int b = j & 1;  // double-buffered: readers of column j - 1 may lag
+      // x = column j below the diagonal: x^T (column q) and, in double, |column q|^2
+      T dot[4] = {T(0), T(0), T(0), T(0)};
+      double nrm[2] = {0.0, 0.0};
+      each([&](int s, M4& v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          T x = row_bcast<j>(v[e]), y = v[e];
+          if (s == 0) {  // rows above the diagonal and on it stay out
+            const bool below = wv > t0 || (wv == t0 && QrMma<T>::row(g, e) > j);
+            x = below ? x : T(0);
+            y = below ? y : T(0);
+          }
+          dot[e] = fma(x, y, dot[e]);
+          if constexpr (sizeof(T) == 4) nrm[e & 1] = fma((double)y, (double)y, nrm[e & 1]);
+        }
+      });
+      T dq = (dot[0] + dot[1]) + (dot[2] + dot[3]);
+      dq += lane_xor<16>(dq);
+      dq += lane_xor<32>(dq);
+      double nq = nrm[0] + nrm[1];
+      if constexpr (sizeof(T) == 4) {
+        nq += lane_xor<16>(nq);
+        nq += lane_xor<32>(nq);
+      }
+      if (g == 0) s_part[b][wv][q] = dq;
+      if (sizeof(T) == 4 && lane == j) s_norm[b][wv] = nq;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (wv == t0 && QrMma<T>::row(g, e) == j) s_diag[b][q] = acc[0][e];
+      lds_barrier();
+      T dots = T(0);
+      double ss = 0.0;
+#pragma unroll
+      for (int i = 0; i < kWaves; ++i) {
+        dots += s_part[b][i][q];
+        ss += sizeof(T) == 4 ? s_norm[b][i] : (double)s_part[b][i][j];
+      }
+      const T dv = s_diag[b][q];
+      const double alpha = (double)s_diag[b][j];
+      T tj = T(0), beta = (T)alpha, scale = T(1);
+      if (ss != 0.0) {
+        const double bd = -copysign(sqrt(alpha * alpha + ss), alpha);
+        beta = (T)bd;
+        tj = (T)((bd - alpha) / bd);
+        scale = (T)(1.0 / (alpha - bd));
+      }
+      // v = [1; scale x]: v^T (column q) for q > j (larf), v_q^T v for q < j
+      // (larft; columns left of j are still unscaled)
+      const T prod = dv + scale * dots;
+      if (tid < j) s_g[tid][j] = sc * prod;
+      if (tid == j) s_tau[j] = tj;
+      if (q == j) sc = scale;
+      // larf on the columns right of j; beta on the diagonal
+      const bool right = q > j && q < nbn;
+      const T on_diag = right ? -tj * prod : T(0);
+      const T coef = on_diag * scale;
+      each([&](int s, M4& v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const T x = row_bcast<j>(v[e]);
+          if (s == 0) {
+            const int r = QrMma<T>::row(g, e);
+            const bool below = wv > t0 || (wv == t0 && r > j);
+            const bool diag = wv == t0 && r == j;
+            const T moved = fma(x, coef, v[e]);
+            v[e] = below ? moved : !diag ? v[e] : q == j ? beta : v[e] + on_diag;
+          } else {
+            v[e] = fma(x, coef, v[e]);
+          }
+        }
+      });
+    });
+    each([&](int s, M4& v) __attribute__((always_inline)) {
+      M4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool below = s > 0 || wv > t0 || (wv == t0 && QrMma<T>::row(g, e) > q);
+        o[e] = below ? v[e] * sc : v[e];
+      }
+      store(s, o);
+    });
+    __syncthreads();  // s_g and s_tau complete
+
+    // ---- T (larft, forward, columnwise): lane a owns row a of T.
+    if (tid < NB) {
+      const int ra = tid;
+      T trow[NB];
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        T v = T(0);
+        if (i < nbn) {
+          if (ra == i) {
+            v = s_tau[i];
+          } else if (ra < i) {
+            T x = T(0);
+#pragma unroll
+            for (int c = 0; c < NB; ++c)
+              if (c >= ra && c < i) x += trow[c] * s_g[c][i];
+            v = -s_tau[i] * x;
+          }
+        }
+        trow[i] = v;
+      }
+      T* Tp = tblk + d.t_offset + (int64_t)(kn / NB) * NB * NB + ra * NB;
+#pragma unroll
+      for (int i = 0; i < NB; ++i) Tp[i] = trow[i];
+      if (ra < nbn) tau[d.tau_offset + kn + ra] = s_tau[ra];
     }
   }
 }
 
-// float32 forms of (1) and (3) on the matrix cores (v_mfma_f32_16x16x4f32,
-// float32 products and accumulation).  Operand layouts (lane l):
-//   A operand: A[l % 16][l / 16];  B operand: B[l / 16][l % 16];
-//   result:    rows 4 (l / 16) + i (i < 4), column l % 16.
-// Each wave of the 256-thread workgroup owns 16 of the block's 64 columns.
-typedef float qr_f4 __attribute__((ext_vector_type(4)));
-
-// (1) W(16 x 16 per wave) = V^T C over one 256-row chunk: A = V^T from LDS,
-// B = C streamed from HBM, four rows per MFMA.  No cross-wave reduction.
-__global__ __launch_bounds__(kTrailThreads) void qr_trail_partial_mfma_kernel(const lxa_qr_desc* __restrict__ descs,
-                                                                            int k_all,
-                                                                            const int32_t* __restrict__ kcol,
-                                                                            const float* __restrict__ a,
-                                                                            float* __restrict__ work) {
-  constexpr int NB = QrCfg<float>::NB;
-  static_assert(NB == 16 && kTrailCols == 64 && kTrailThreads == 256, "one 16-column slab per wave");
-  __shared__ float sv[kTrailRows][NB];
-  const lxa_qr_desc d = descs[blockIdx.z];
-  const int m = d.m, n = d.n, lda = d.lda;
-  const int kmax = min(m, n);
-  const int k = kcol ? kcol[blockIdx.z] : k_all;
-  if (k >= kmax) return;
-  const int nb = min(NB, kmax - k);
-  const int c0 = k + nb + kTrailCols * (int)blockIdx.x;
-  const int r0 = k + kTrailRows * (int)blockIdx.y;
-  if (c0 >= n || r0 >= m) return;
-  const int tid = threadIdx.x, l = tid & (kWave - 1), wv = tid >> 6;
-  const float* A = a + d.a_offset;
-  load_v_chunk<float, NB>(sv, A, lda, m, k, nb, r0, tid);
-  __syncthreads();
-  const int col = c0 + 16 * wv + (l & 15);
-  const bool cv = col < n;
-  const int rows = min(kTrailRows, m - r0);
-  qr_f4 acc = {0.f, 0.f, 0.f, 0.f};
-  // rows kk + l / 16 of the chunk; eight MFMA row groups (32 rows) per batch
-  constexpr int kGroups = 8;
-  for (int kb = 0; kb < rows; kb += 4 * kGroups) {
-    float cb[kGroups];
-#pragma unroll
-    for (int u = 0; u < kGroups; ++u) {
-      const int i = kb + 4 * u + (l >> 4);
-      cb[u] = (cv && i < rows) ? A[(int64_t)(r0 + i) * lda + col] : 0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < kGroups; ++u) {
-      const int i = kb + 4 * u + (l >> 4);
-      const float av = i < kTrailRows ? sv[i][l & 15] : 0.f;  // zero past the chunk (and past m)
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, cb[u], acc, 0, 0, 0);
-    }
+template <typename T, int KR, int KL>
+int launch_step(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int mode, int k, const int32_t* kcol,
+                int blocks, T* a, T* tau, T* tblk) {
+  const size_t smem = sizeof(T) * (size_t)KL * 4 * kPanelThreads;
+  if (smem) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&qr_step_kernel<T, KR, KL>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return hip_error(e, "hipFuncSetAttribute(qr_step_kernel)");
   }
-  float* W = work + d.w_offset + (int64_t)blockIdx.y * NB * n;
-  if (cv) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) W[(int64_t)(4 * (l >> 4) + i) * n + col] = acc[i];
+  // a grid holds fewer than 2^32 threads: launches of at most 2^22 workgroups
+  // of 512, whole column blocks of systems at a time
+  const int64_t chunk = std::max<int64_t>(1, (int64_t(1) << 22) / blocks);
+  for (int64_t s0 = 0; s0 < count; s0 += chunk) {
+    const int64_t cnt = std::min(chunk, count - s0);
+    qr_step_kernel<T, KR, KL><<<dim3((unsigned)(cnt * blocks)), kPanelThreads, smem, st>>>(
+        desc + s0, cnt, mode, k, kcol ? kcol + s0 : nullptr, a, tau, tblk);
   }
+  LXA_LAUNCH_CHECK("qr_step_kernel");
+  return LXA_OK;
 }
 
-// (3) C -= V W: each wave takes its 16 columns down the chunk in 16 x 16
-// tiles; the tile is loaded into the accumulator, and V (from LDS) times -W
-// (registers) is added by four MFMAs.
-__global__ __launch_bounds__(kTrailThreads) void qr_trail_update_mfma_kernel(const lxa_qr_desc* __restrict__ descs,
-                                                                           int k_all,
-                                                                           const int32_t* __restrict__ kcol,
-                                                                           float* __restrict__ a,
-                                                                           const float* __restrict__ work) {
-  constexpr int NB = QrCfg<float>::NB;
-  __shared__ float sv[kTrailRows][NB];
-  const lxa_qr_desc d = descs[blockIdx.z];
-  const int m = d.m, n = d.n, lda = d.lda;
-  const int kmax = min(m, n);
-  const int k = kcol ? kcol[blockIdx.z] : k_all;
-  if (k >= kmax) return;
-  const int nb = min(NB, kmax - k);
-  const int c0 = k + nb + kTrailCols * (int)blockIdx.x;
-  const int r0 = k + kTrailRows * (int)blockIdx.y;
-  if (c0 >= n || r0 >= m) return;
-  const int tid = threadIdx.x, l = tid & (kWave - 1), wv = tid >> 6;
-  float* A = a + d.a_offset;
-  load_v_chunk<float, NB>(sv, A, lda, m, k, nb, r0, tid);
-  const int col = c0 + 16 * wv + (l & 15);
-  const bool cv = col < n;
-  // -W as the B operand: rows j = 4 s + l / 16 of this wave's columns
-  const float* W = work + d.w_offset;
-  float wb[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) wb[q] = cv ? -W[(int64_t)(4 * q + (l >> 4)) * n + col] : 0.f;
-  __syncthreads();
-  const int rows = min(kTrailRows, m - r0);
-  for (int rt = 0; rt < rows; rt += 16) {
-    qr_f4 acc;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = rt + 4 * (l >> 4) + i;
-      acc[i] = (cv && row < rows) ? A[(int64_t)(r0 + row) * lda + col] : 0.f;
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float av = sv[rt + (l & 15)][4 * q + (l >> 4)];
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, wb[q], acc, 0, 0, 0);
-    }
-    if (cv) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = rt + 4 * (l >> 4) + i;
-        if (row < rows) A[(int64_t)(r0 + row) * lda + col] = acc[i];
-      }
-    }
+// rows bounds m - k over the systems; blocks is the number of 16-column blocks.
+template <typename T>
+int step(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int mode, int k, const int32_t* kcol, int rows,
+         int blocks, T* a, T* tau, T* tblk) {
+  if (rows <= 512) return launch_step<T, 4, 0>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
+  if (rows <= 1024) return launch_step<T, 8, 0>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
+  if (rows <= 2048) return launch_step<T, 16, 0>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
+  if constexpr (sizeof(T) == 4) {
+    if (rows <= kStepMaxRows) return launch_step<T, 24, 8>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
+  } else {
+    if (rows <= 3072) return launch_step<T, 16, 8>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
+    if (rows <= kStepMaxRows) return launch_step<T, 24, 8>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
   }
+  return launch_step<T, 0, 0>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
 }
 
 // ---------------------------------------------------------------------------
@@ -966,53 +968,44 @@ size_t trsv_smem_bytes(int dtype) {
   return e * (((kTrsvMaxK + 1) & ~1) + kTrsvBlock * (kTrsvBlock + 1) + kBigWaves * kWave + kTrsvBlock);
 }
 
-// One panel step for every system: column k_all for all (kcol == nullptr)
-// or kcol[s] for system s.  max_rows bounds m - k and max_trail_cols bounds
-// n - k - 1 over the systems that still have columns.
+// Panels at column k_all (kcol == nullptr) or kcol[s] for system s.  max_rows
+// bounds m - k over the systems that still have columns.
 template <typename T>
-int qr_step_impl(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int k_all, const int32_t* kcol,
-                 int max_rows, int max_trail_cols, T* a, T* tau, T* tblk, T* work) {
-  const int rpt = (max_rows + kPanelThreads - 1) / kPanelThreads;
-  const dim3 pg((unsigned)count);
-  if (rpt <= 1)
-    qr_panel_kernel<T, 1><<<pg, kPanelThreads, 0, st>>>(desc, k_all, kcol, a, tau, tblk);
-  else if (rpt <= 2)
-    qr_panel_kernel<T, 2><<<pg, kPanelThreads, 0, st>>>(desc, k_all, kcol, a, tau, tblk);
-  else if (rpt <= 4)
-    qr_panel_kernel<T, 4><<<pg, kPanelThreads, 0, st>>>(desc, k_all, kcol, a, tau, tblk);
-  else if (rpt <= kPanelMaxRpt)
-    qr_panel_kernel<T, kPanelMaxRpt><<<pg, kPanelThreads, 0, st>>>(desc, k_all, kcol, a, tau, tblk);
-  else
-    qr_panel_kernel<T, 0><<<pg, kPanelThreads, 0, st>>>(desc, k_all, kcol, a, tau, tblk);
+int panel_only(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int k_all, const int32_t* kcol, int max_rows,
+               T* a, T* tau, T* tblk) {
+  if (max_rows <= kStepMaxRows) return step<T>(st, count, desc, kStepPanel, k_all, kcol, max_rows, 1, a, tau, tblk);
+  qr_panel_kernel<T><<<dim3((unsigned)count), kPanelThreads, 0, st>>>(desc, k_all, kcol, a, tau, tblk);
   LXA_LAUNCH_CHECK("qr_panel_kernel");
-  if (max_trail_cols <= 0) return LXA_OK;
-  const unsigned cb = (unsigned)((max_trail_cols + kTrailCols - 1) / kTrailCols);
-  const unsigned rc = (unsigned)((max_rows + kTrailRows - 1) / kTrailRows);
-  if constexpr (std::is_same_v<T, float>) {
-    qr_trail_partial_mfma_kernel<<<dim3(cb, rc, (unsigned)count), kTrailThreads, 0, st>>>(desc, k_all, kcol, a,
-                                                                                          work);
-  } else {
-    qr_trail_partial_kernel<T><<<dim3(cb, rc, (unsigned)count), kTrailThreads, 0, st>>>(desc, k_all, kcol, a, work);
-  }
-  LXA_LAUNCH_CHECK("qr_trail_partial_kernel");
-  qr_trail_reduce_kernel<T><<<dim3(cb, (unsigned)count), kTrailThreads, 0, st>>>(desc, k_all, kcol, tblk, work);
-  LXA_LAUNCH_CHECK("qr_trail_reduce_kernel");
-  if constexpr (std::is_same_v<T, float>) {
-    qr_trail_update_mfma_kernel<<<dim3(cb, rc, (unsigned)count), kTrailThreads, 0, st>>>(desc, k_all, kcol, a,
-                                                                                         work);
-  } else {
-    qr_trail_update_kernel<T><<<dim3(cb, rc, (unsigned)count), kTrailThreads, 0, st>>>(desc, k_all, kcol, a, work);
-  }
-  LXA_LAUNCH_CHECK("qr_trail_update_kernel");
   return LXA_OK;
+}
+
+// One panel step for every system: factor the panel, update the columns right
+// of it.  max_trail_cols bounds n - k - 1.
+template <typename T>
+int qr_step_impl(hipStream_t st, int64_t count, const lxa_qr_desc* desc, const int32_t* kcol, int max_rows,
+                 int max_trail_cols, T* a, T* tau, T* tblk) {
+  if (int rc = panel_only<T>(st, count, desc, 0, kcol, max_rows, a, tau, tblk)) return rc;
+  if (max_trail_cols <= 0) return LXA_OK;
+  return step<T>(st, count, desc, kStepUpdate, 0, kcol, max_rows, (max_trail_cols + 15) / 16, a, tau, tblk);
 }
 
 template <typename T>
 int qr_factor_impl(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int max_m, int max_n, int max_k, T* a,
-                   T* tau, T* tblk, T* work) {
+                   T* tau, T* tblk) {
   constexpr int NB = QrCfg<T>::NB;
+  if (int rc = panel_only<T>(st, count, desc, 0, nullptr, max_m, a, tau, tblk)) return rc;
   for (int k = 0; k < max_k; k += NB) {
-    if (int rc = qr_step_impl<T>(st, count, desc, k, nullptr, max_m - k, max_n - k - 1, a, tau, tblk, work)) return rc;
+    // columns right of the panel: past it by its width, 1..16 columns
+    const int right = max_n - k - 1;
+    if (right <= 0) break;
+    const int rows = max_m - k;
+    const bool ahead = rows <= kStepMaxRows;
+    if (int rc = step<T>(st, count, desc, ahead ? kStepLookahead : kStepUpdate, k, nullptr, rows, (right + 15) / 16, a,
+                         tau, tblk))
+      return rc;
+    if (!ahead && k + NB < max_k) {
+      if (int rc = panel_only<T>(st, count, desc, k + NB, nullptr, rows - NB, a, tau, tblk)) return rc;
+    }
   }
   return LXA_OK;
 }
@@ -1034,8 +1027,7 @@ extern "C" int lxa_qr_block(int dtype) { return dtype == LXA_F64 ? QrCfg<double>
 extern "C" int lxa_qr_work_elems(int dtype, int64_t m, int64_t n, int64_t* elems) {
   LXA_REQUIRE(dtype == LXA_F32 || dtype == LXA_F64, "dtype must be LXA_F32 or LXA_F64 (got %d)", dtype);
   LXA_REQUIRE(m >= 0 && n >= 0 && elems != nullptr, "invalid arguments");
-  const int64_t nb = lxa_qr_block(dtype);
-  *elems = ((m + kTrailRows - 1) / kTrailRows) * nb * n;
+  *elems = 1;  // nothing is used: the smallest buffer that is one
   return LXA_OK;
 }
 
@@ -1049,9 +1041,9 @@ extern "C" int lxa_qr_factor(void* stream, int dtype, int64_t count, const lxa_q
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == LXA_F32)
     return qr_factor_impl<float>(st, count, desc, max_m, max_n, max_k, static_cast<float*>(a),
-                                 static_cast<float*>(tau), static_cast<float*>(tblk), static_cast<float*>(work));
+                                 static_cast<float*>(tau), static_cast<float*>(tblk));
   return qr_factor_impl<double>(st, count, desc, max_m, max_n, max_k, static_cast<double*>(a),
-                                static_cast<double*>(tau), static_cast<double*>(tblk), static_cast<double*>(work));
+                                static_cast<double*>(tau), static_cast<double*>(tblk));
 }
 
 extern "C" int lxa_qr_factor_step(void* stream, int dtype, int64_t count, const lxa_qr_desc* desc,
@@ -1064,10 +1056,10 @@ extern "C" int lxa_qr_factor_step(void* stream, int dtype, int64_t count, const 
   LXA_REQUIRE(a && tau && tblk && work, "a, tau, tblk and work must be non-NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == LXA_F32)
-    return qr_step_impl<float>(st, count, desc, 0, kcol, max_rows, max_trail_cols, static_cast<float*>(a),
-                               static_cast<float*>(tau), static_cast<float*>(tblk), static_cast<float*>(work));
-  return qr_step_impl<double>(st, count, desc, 0, kcol, max_rows, max_trail_cols, static_cast<double*>(a),
-                              static_cast<double*>(tau), static_cast<double*>(tblk), static_cast<double*>(work));
+    return qr_step_impl<float>(st, count, desc, kcol, max_rows, max_trail_cols, static_cast<float*>(a),
+                               static_cast<float*>(tau), static_cast<float*>(tblk));
+  return qr_step_impl<double>(st, count, desc, kcol, max_rows, max_trail_cols, static_cast<double*>(a),
+                              static_cast<double*>(tau), static_cast<double*>(tblk));
 }
 
 extern "C" int lxa_qr_apply(void* stream, int dtype, int64_t count, const lxa_qr_desc* desc, int max_m, int max_k,

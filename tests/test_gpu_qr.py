@@ -65,6 +65,45 @@ def test_geqrf_f32_close_to_f64(device, rng, shape):
     assert np.max(np.abs(r_got - r_ref)) <= tol * np.max(np.abs(r_ref))
 
 
+@pytest.mark.parametrize("shape", [(15, 15), (512, 33), (513, 33), (528, 17), (1025, 40), (2049, 31), (2064, 40),
+                                   (3073, 20), (3100, 50), (4096, 18), (4097, 18), (4112, 33), (18, 530), (40, 71)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_geqrf_step_edges(device, rng, shape, dtype):
+    """Heights around the step kernel's tiles and register / LDS limits, widths
+    that leave partial panels, wide matrices, three systems with one of them
+    rank deficient.
+
+    Bounds: column j of A - Q R is below m n u |a_j| and Q^T Q - I below m n u
+    (Higham, Accuracy and Stability, thm 19.4 with c = 1), the compact-WY blocks
+    to the same."""
+    m, n = shape
+    k = min(m, n)
+    u = torch.finfo(dtype).eps / 2
+    mats = rng.standard_normal((3, m, n))
+    mats[1] *= 10.0 ** rng.uniform(-6, 6, size=n)
+    mats[2, :, k // 2] = 0.0
+    t = _t(mats, device, dtype)
+    ad, tau, tblk = K.qr_factor(t)
+    exact = t.cpu().double().numpy()
+    h, tau, tblk = ad.cpu().double().numpy(), tau.cpu().double().numpy(), tblk.cpu().double().numpy()
+    assert tau[2, k // 2] == 0.0 or np.abs(h[2, k // 2:, k // 2]).max() < 1.0
+    nb = tblk.shape[-1]
+    for i in range(3):
+        v = np.tril(h[i][:, :k], -1) + np.eye(m, k)
+        q = np.eye(m, k)
+        for j in reversed(range(k)):
+            q -= tau[i, j] * np.outer(v[:, j], v[:, j] @ q)
+        r = np.triu(h[i][:k])
+        err = np.linalg.norm(exact[i] - q @ r, axis=0)
+        assert np.all(err <= m * n * u * np.linalg.norm(exact[i], axis=0))
+        assert np.linalg.norm(q.T @ q - np.eye(k), 2) <= m * n * u
+        wy = np.eye(m, k)
+        for p in reversed(range(tblk.shape[1])):
+            vp = v[:, p * nb: p * nb + nb]
+            wy -= vp @ (tblk[i, p][: vp.shape[1], : vp.shape[1]] @ (vp.T @ wy))
+        assert np.linalg.norm(wy - q, 2) <= m * n * u
+
+
 def test_geqrf_zero_column_gives_zero_tau(device):
     a = np.zeros((6, 3))
     a[:, 1] = np.arange(6) + 1.0
