@@ -3,9 +3,6 @@
 // Three tiers, chosen by order n:
 //  * n <= 64: one lane per row in registers, 64/LPS systems per wave; the
 //    scaled pivot row is broadcast through a double-buffered LDS row.
-//  * n <= 256, float factors: the register-tiled 16-column panel
-//    factorisation of chol_uneven.hip (chol_factor_regs_f32), one workgroup
-//    per system.
 //  * n <= 256 (float) / 181 (double) solves, and double factors of many small
 //    systems: one 256-thread workgroup per system with the upper triangle in
 //    LDS in row-packed form (131.6 KB at n = 256): right-looking
@@ -373,10 +370,7 @@ int chol_factor_t(hipStream_t s, int64_t batch, int64_t n64, T* a, int64_t strid
   else if (n <= 16) launch_chol_small<T, 16>(s, batch, n, a, stride, negate, info);
   else if (n <= 32) launch_chol_small<T, 32>(s, batch, n, a, stride, negate, info);
   else if (n <= 64) launch_chol_small<T, 64>(s, batch, n, a, stride, negate, info);
-  else if (sizeof(T) == 4 && n <= 256) {
-    // register-tiled 16-column panels (chol_uneven.hip)
-    return chol_factor_regs_f32(s, batch, n, reinterpret_cast<float*>(a), stride, negate, info);
-  } else if (n <= kLdsFactorMax && batch > kLdsFactorBatch) {
+  else if (sizeof(T) == 8 && n <= kLdsFactorMax && batch > kLdsFactorBatch) {
     const size_t shmem = static_cast<size_t>(n) * (n + 1) / 2 * sizeof(T);
     if (int rc = allow_lds(chol_factor_lds_kernel<T>, shmem)) return rc;
     hipLaunchKernelGGL((chol_factor_lds_kernel<T>), dim3(static_cast<unsigned>(batch)), dim3(kWG), shmem, s, n, a,

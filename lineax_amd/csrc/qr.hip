@@ -271,16 +271,43 @@ struct QrMma<double> {
 
 // The value of lane J of this lane's row of 16 (DPP row_newbcast; every lane
 // must be active).
-template <int J>
-__device__ __forceinline__ float row_bcast(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + J, 0xF, 0xF, false));
+template <int J, typename T>
+__device__ __forceinline__ T row_bcast(T v) {
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x150 + J, 0xF, 0xF, true));
+  } else {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_mov_dpp(static_cast<int>(u), 0x150 + J, 0xF, 0xF, true);
+    const uint32_t hi = __builtin_amdgcn_mov_dpp(static_cast<int>(u >> 32), 0x150 + J, 0xF, 0xF, true);
+    return __builtin_bit_cast(T, (static_cast<uint64_t>(hi) << 32) | lo);
+  }
 }
-template <int J>
-__device__ __forceinline__ double row_bcast(double v) {
-  const uint64_t u = static_cast<uint64_t>(__double_as_longlong(v));
-  const uint32_t lo = __builtin_amdgcn_update_dpp(0u, static_cast<uint32_t>(u), 0x150 + J, 0xF, 0xF, false);
-  const uint32_t hi = __builtin_amdgcn_update_dpp(0u, static_cast<uint32_t>(u >> 32), 0x150 + J, 0xF, 0xF, false);
-  return __longlong_as_double(static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo));
+
+// larfg in double: from alpha and the squared norm ss > 0 below it, beta =
+// -sign(alpha) |[alpha; x]|, tau = (beta - alpha) / beta and 1 / (alpha - beta).
+// Every wave repeats it for every column, so the instructions count: hardware
+// reciprocals and Newton steps to full precision, a third of the operations
+// of a square root and two divisions.
+__device__ __forceinline__ void reflector(double alpha, double ss, double& beta, double& tau, double& scale) {
+  const double t = fma(alpha, alpha, ss);
+  if (t >= 0x1p-800 && t <= 0x1p800) {  // uniform
+    double r = __builtin_amdgcn_rsq(t);
+    r = fma(r, fma(-t * r, 0.5 * r, 0.5), r);
+    r = fma(r, fma(-t * r, 0.5 * r, 0.5), r);
+    double norm = t * r;
+    norm = fma(fma(-norm, norm, t), 0.5 * r, norm);
+    const double den = fabs(alpha) + norm;
+    double c = __builtin_amdgcn_rcp(den);
+    c = fma(fma(-den, c, 1.0), c, c);
+    c = fma(fma(-den, c, 1.0), c, c);
+    beta = -copysign(norm, alpha);
+    tau = den * r;  // 1 + |alpha| / norm
+    scale = copysign(c, alpha);
+  } else {
+    beta = -copysign(sqrt(t), alpha);
+    tau = (beta - alpha) / beta;
+    scale = 1.0 / (alpha - beta);
+  }
 }
 
 // What a launch does with the panel at column k.
@@ -374,6 +401,22 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
       for (int e = 0; e < 4; ++e) far[e * kPanelThreads] = v[e];
     }
   };
+  auto each_read = [&](auto&& f) __attribute__((always_inline)) {
+    static_for<0, KR / 4>([&](auto G_) __attribute__((always_inline)) {
+      constexpr int s4 = 4 * decltype(G_)::value;
+      if (s4 < ns) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) f(s4 + u, acc[s4 + u]);
+      }
+    });
+    for (int s = KR; s < (KL > 0 ? ns : 0); ++s) {
+      const T* far = far_slots + (int64_t)(s - KR) * 4 * kPanelThreads + tid;
+      M4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = far[e * kPanelThreads];
+      f(s, v);
+    }
+  };
   if constexpr (KR > 0) each([&](int s, M4& v) __attribute__((always_inline)) { v = load(s); });
 
   if (mode != kStepPanel) {
@@ -397,7 +440,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
     };
     M4 w = {T(0), T(0), T(0), T(0)};
     if constexpr (KR > 0) {
-      each([&](int s, M4& v) __attribute__((always_inline)) { w = project(s, v, w); });
+      each_read([&](int s, const M4& v) __attribute__((always_inline)) { w = project(s, v, w); });
     } else {
 #pragma unroll 4
       for (int s = 0; s < ns; ++s) w = project(s, load(s), w);
@@ -442,7 +485,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
   if constexpr (KR > 0) {
     const int kn = mode == kStepPanel ? k : k + NB;  // the panel to factor
     if (mode == kStepUpdate || blk != 0 || kn >= kmax) {
-      each([&](int s, M4& v) __attribute__((always_inline)) { store(s, v); });
+      each_read([&](int s, const M4& v) __attribute__((always_inline)) { store(s, v); });
       return;
     }
     const int nbn = min(NB, kmax - kn);
@@ -455,17 +498,17 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
       // x = column j below the diagonal: x^T (column q) and, in double, |column q|^2
       T dot[4] = {T(0), T(0), T(0), T(0)};
       double nrm[2] = {0.0, 0.0};
-      each([&](int s, M4& v) __attribute__((always_inline)) {
+      each_read([&](int s, const M4& v) __attribute__((always_inline)) {
+        if (s == 0 && wv < t0) return;  // uniform: rows above the panel
+        M4 y = v;
+        if (s == 0 && wv == t0) {       // uniform: rows above the diagonal and on it stay out
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[e] = QrMma<T>::row(g, e) > j ? v[e] : T(0);
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          T x = row_bcast<j>(v[e]), y = v[e];
-          if (s == 0) {  // rows above the diagonal and on it stay out
-            const bool below = wv > t0 || (wv == t0 && QrMma<T>::row(g, e) > j);
-            x = below ? x : T(0);
-            y = below ? y : T(0);
-          }
-          dot[e] = fma(x, y, dot[e]);
-          if constexpr (sizeof(T) == 4) nrm[e & 1] = fma((double)y, (double)y, nrm[e & 1]);
+          dot[e] = fma(row_bcast<j>(y[e]), y[e], dot[e]);
+          if constexpr (sizeof(T) == 4) nrm[e & 1] = fma((double)y[e], (double)y[e], nrm[e & 1]);
         }
       });
       T dq = (dot[0] + dot[1]) + (dot[2] + dot[3]);
@@ -478,9 +521,8 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
       }
       if (g == 0) s_part[b][wv][q] = dq;
       if (sizeof(T) == 4 && lane == j) s_norm[b][wv] = nq;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (wv == t0 && QrMma<T>::row(g, e) == j) s_diag[b][q] = acc[0][e];
+      constexpr int gj = sizeof(T) == 4 ? j / 4 : j % 4, ej = sizeof(T) == 4 ? j % 4 : j / 4;  // row(gj, ej) = j
+      if (wv == t0 && g == gj) s_diag[b][q] = acc[0][ej];
       lds_barrier();
       T dots = T(0);
       double ss = 0.0;
@@ -493,10 +535,11 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
       const double alpha = (double)s_diag[b][j];
       T tj = T(0), beta = (T)alpha, scale = T(1);
       if (ss != 0.0) {
-        const double bd = -copysign(sqrt(alpha * alpha + ss), alpha);
+        double bd, td, sd;
+        reflector(alpha, ss, bd, td, sd);
         beta = (T)bd;
-        tj = (T)((bd - alpha) / bd);
-        scale = (T)(1.0 / (alpha - bd));
+        tj = (T)td;
+        scale = (T)sd;
       }
       // v = [1; scale x]: v^T (column q) for q > j (larf), v_q^T v for q < j
       // (larft; columns left of j are still unscaled)
@@ -509,22 +552,21 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
       const T on_diag = right ? -tj * prod : T(0);
       const T coef = on_diag * scale;
       each([&](int s, M4& v) __attribute__((always_inline)) {
+        if (s == 0 && wv < t0) return;  // uniform
+        if (s == 0 && wv == t0) {       // uniform
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const T x = row_bcast<j>(v[e]);
-          if (s == 0) {
-            const int r = QrMma<T>::row(g, e);
-            const bool below = wv > t0 || (wv == t0 && r > j);
-            const bool diag = wv == t0 && r == j;
-            const T moved = fma(x, coef, v[e]);
-            v[e] = below ? moved : !diag ? v[e] : q == j ? beta : v[e] + on_diag;
-          } else {
-            v[e] = fma(x, coef, v[e]);
+          for (int e = 0; e < 4; ++e) {
+            const T moved = fma(row_bcast<j>(v[e]), coef, v[e]);
+            v[e] = QrMma<T>::row(g, e) > j ? moved : v[e];
           }
+          if (g == gj) acc[0][ej] = q == j ? beta : acc[0][ej] + on_diag;
+          return;
         }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = fma(row_bcast<j>(v[e]), coef, v[e]);
       });
     });
-    each([&](int s, M4& v) __attribute__((always_inline)) {
+    each_read([&](int s, const M4& v) __attribute__((always_inline)) {
       M4 o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
