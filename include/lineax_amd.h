@@ -631,6 +631,11 @@ int lxa_chol_blocked_solve(void* stream, int64_t count, const lxa_qr_desc* desc,
  * The caller advances kcol by the block after the call. */
 int lxa_qr_factor_step(void* stream, int dtype, int64_t count, const lxa_qr_desc* desc, const int32_t* kcol,
                        int max_rows, int max_trail_cols, void* a, void* tau, void* tblk, void* work);
+/* `steps` of them in one call, from column kcol[s] of each system on (kcol is
+ * not changed; max_rows and max_trail_cols are those of the first step): each
+ * step's update factors the panel of the next. */
+int lxa_qr_factor_steps(void* stream, int dtype, int64_t count, const lxa_qr_desc* desc, const int32_t* kcol, int steps,
+                        int max_rows, int max_trail_cols, void* a, void* tau, void* tblk, void* work);
 /* b <- Q^T b (trans = 1, ormqr with transpose=True, qr.py:89) or b <- Q b
  * (trans = 0, the min-norm branch's ormqr, qr.py:86) for vectors of length m. */
 int lxa_qr_apply(void* stream, int dtype, int64_t count, const lxa_qr_desc* desc, int max_m, int max_k,

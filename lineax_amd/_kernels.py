@@ -113,6 +113,7 @@ _SIGNATURES = {
     "lxa_qr_factor": [_vp, _int, _i64, _vp, _int, _int, _int, _vp, _vp, _vp, _vp],
     "lxa_qr_apply": [_vp, _int, _i64, _vp, _int, _int, _vp, _vp, _int, _vp, _int],
     "lxa_qr_factor_step": [_vp, _int, _i64, _vp, _vp, _int, _int, _vp, _vp, _vp, _vp],
+    "lxa_qr_factor_steps": [_vp, _int, _i64, _vp, _vp, _int, _int, _int, _vp, _vp, _vp, _vp],
     "lxa_chol_blocked_factor": [_vp, _i64, _vp, _vp, _vp],
     "lxa_chol_blocked_solve": [_vp, _i64, _vp, _vp, _vp],
     "lxa_trsv": [_vp, _int, _i64, _vp, _int, _vp, _int, _vp, _int, _int, _int],
@@ -781,16 +782,17 @@ def qr_factor_raw(descs: torch.Tensor, count: int, max_m: int, max_n: int, max_k
 
 
 def qr_factor_step_raw(descs: torch.Tensor, count: int, kcol: torch.Tensor, max_rows: int, max_trail_cols: int,
-                       a: torch.Tensor, tau: torch.Tensor, tblk: torch.Tensor, work: torch.Tensor) -> None:
-    """One panel step of every system at its own column kcol[s] (int32, device)."""
+                       a: torch.Tensor, tau: torch.Tensor, tblk: torch.Tensor, work: torch.Tensor,
+                       steps: int = 1) -> None:
+    """``steps`` panel steps of every system from its own column kcol[s] (int32, device) on."""
     for t, what in ((descs, "descs"), (kcol, "kcol"), (a, "a"), (tau, "tau"), (tblk, "tblk"), (work, "work")):
         _gpu(t, what)
     if kcol.dtype != torch.int32:
         raise TypeError("kcol must be int32")
     _check(
-        load().lxa_qr_factor_step(_stream(a), _dtype_code(a.dtype), int(count), _ptr(descs), _ptr(kcol),
-                                  int(max_rows), int(max_trail_cols), _ptr(a), _ptr(tau), _ptr(tblk), _ptr(work)),
-        "lxa_qr_factor_step",
+        load().lxa_qr_factor_steps(_stream(a), _dtype_code(a.dtype), int(count), _ptr(descs), _ptr(kcol), int(steps),
+                                   int(max_rows), int(max_trail_cols), _ptr(a), _ptr(tau), _ptr(tblk), _ptr(work)),
+        "lxa_qr_factor_steps",
     )
 
 

@@ -130,7 +130,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_panel_kernel(const lxa_qr_de
   const lxa_qr_desc d = descs[blockIdx.x];
   const int m = d.m, n = d.n, lda = d.lda;
   const int kmax = min(m, n);
-  const int k = kcol ? kcol[blockIdx.x] : k_all;
+  const int k = (kcol ? kcol[blockIdx.x] : 0) + k_all;
   if (k >= kmax) return;
   const int nb = min(NB, kmax - k);
   const int tid = threadIdx.x;
@@ -269,6 +269,34 @@ struct QrMma<double> {
   static __device__ __forceinline__ constexpr int row(int g, int e) { return g + 4 * e; }
 };
 
+// The 64-bit move (one instruction instead of two); the builtin takes 64-bit
+// values only with literal controls, hence the switch (j is a constant).
+__device__ __forceinline__ long long row_bcast64(long long v, int j) {
+#define LXA_ROW_BCAST(J) \
+  case J:                \
+    return __builtin_amdgcn_update_dpp(v, v, 0x150 + J, 0xF, 0xF, true);
+  switch (j) {
+    LXA_ROW_BCAST(0)
+    LXA_ROW_BCAST(1)
+    LXA_ROW_BCAST(2)
+    LXA_ROW_BCAST(3)
+    LXA_ROW_BCAST(4)
+    LXA_ROW_BCAST(5)
+    LXA_ROW_BCAST(6)
+    LXA_ROW_BCAST(7)
+    LXA_ROW_BCAST(8)
+    LXA_ROW_BCAST(9)
+    LXA_ROW_BCAST(10)
+    LXA_ROW_BCAST(11)
+    LXA_ROW_BCAST(12)
+    LXA_ROW_BCAST(13)
+    LXA_ROW_BCAST(14)
+    LXA_ROW_BCAST(15)
+  }
+#undef LXA_ROW_BCAST
+  return v;
+}
+
 // The value of lane J of this lane's row of 16 (DPP row_newbcast; every lane
 // must be active).
 template <int J, typename T>
@@ -276,10 +304,7 @@ __device__ __forceinline__ T row_bcast(T v) {
   if constexpr (sizeof(T) == 4) {
     return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x150 + J, 0xF, 0xF, true));
   } else {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = __builtin_amdgcn_mov_dpp(static_cast<int>(u), 0x150 + J, 0xF, 0xF, true);
-    const uint32_t hi = __builtin_amdgcn_mov_dpp(static_cast<int>(u >> 32), 0x150 + J, 0xF, 0xF, true);
-    return __builtin_bit_cast(T, (static_cast<uint64_t>(hi) << 32) | lo);
+    return __builtin_bit_cast(T, row_bcast64(__builtin_bit_cast(long long, v), J));
   }
 }
 
@@ -317,14 +342,33 @@ enum : int {
   kStepLookahead = 2,  // apply it, and factor the panel after it
 };
 
+// Columns of a workgroup that does not keep them in registers: V is read once
+// per 64 columns instead of once per 16.
+constexpr int kWideTiles = 4;
+constexpr int kWideCols = 16 * kWideTiles;
+constexpr int kWideLd = kWideCols + 1;
+
+// Column blocks of a launch that updates `right` columns.  All blocks of a
+// KR = 4 lookahead launch (panels of up to 512 rows) have 16 columns in
+// registers; taller ones have the next panel's 16 and wide blocks after it.
+constexpr bool step_wide(int KR, int mode) { return mode == kStepUpdate || KR > 4; }
+inline int step_blocks(int KR, int mode, int right) {
+  if (mode == kStepPanel) return 1;
+  if (mode == kStepUpdate) return (right + kWideCols - 1) / kWideCols;
+  if (!step_wide(KR, mode)) return (right + 15) / 16;
+  return 1 + (std::max(0, right - 16) + kWideCols - 1) / kWideCols;
+}
+
 // KR: 16-row tiles per wave held in registers (slot s of wave w is tile
 // w + 8 s of the rows from k on); KL: further ones in LDS (the register file
-// holds 2048 double or 3072 float rows beside what the products need).  KR = 0: any height, C read again for the update; no panel.
+// holds 2048 double or 3072 float rows beside what the products need).
+// KR = 0: wide blocks only, any height.
 template <typename T, int KR, int KL>
 __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_desc* __restrict__ descs, int64_t count,
                                                                 int mode, int k_all,
                                                                 const int32_t* __restrict__ kcol, T* __restrict__ a,
                                                                 T* __restrict__ tau, T* __restrict__ tblk) {
+  // the panel's column: k_all, past kcol[s] where that is given
   constexpr int NB = QrCfg<T>::NB;
   static_assert(NB == 16 && KR % 4 == 0, "16-column panels; slots go in groups of four");
   constexpr int kWaves = kPanelWaves, kSpan = 16 * kWaves;  // rows per slot over the waves
@@ -343,10 +387,14 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
   const lxa_qr_desc d = descs[sys];
   const int m = d.m, n = d.n, lda = d.lda;
   const int kmax = min(m, n);
-  const int k = kcol ? kcol[sys] : k_all;
+  const int k = (kcol ? kcol[sys] : 0) + k_all;
   if (k >= kmax) return;
   const int nb = min(NB, kmax - k);
-  const int c0 = mode == kStepPanel ? k : k + nb + NB * blk;
+  const bool wide = mode == kStepUpdate || (mode == kStepLookahead && KR > 4 && blk > 0);
+  const int c0 = mode == kStepPanel      ? k
+                 : mode == kStepUpdate   ? k + nb + kWideCols * blk
+                 : KR > 4 && blk > 0     ? k + nb + 16 + kWideCols * (blk - 1)
+                                         : k + nb + 16 * blk;
   if (c0 >= n) return;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q = lane & 15, g = lane >> 4;
@@ -366,6 +414,100 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
   }
   auto base = [&](int s) { return A + (int64_t)min(k + kSpan * s, m - 1) * lda; };  // uniform
   auto exists = [&](int s, int e) { return kSpan * s + rel[e] < rows; };
+  // T^T as the A operand of T^T W; rows of V as the A operands of V^T C
+  // (project_v) and of V (T^T W) (expand_v)
+  T tt[4] = {T(0), T(0), T(0), T(0)};
+  if (mode != kStepPanel) {
+    const T* Tp = tblk + d.t_offset + (int64_t)(k / NB) * NB * NB;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tt[e] = Tp[QrMma<T>::row(g, e) * NB + q];
+  }
+  auto project_v = [&](int s, T (&x)[4]) {
+    const T* p = base(s) + k + min(q, nb - 1);
+    T v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = p[exists(s, e) ? off[e] : 0];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = exists(s, e) && q < nb ? vpick(kSpan * s + rel[e], q, v[e]) : T(0);
+  };
+  const int rq = 16 * wv + q;
+  const int64_t offq = (int64_t)rq * lda;
+  auto expand_v = [&](int s, T (&x)[4]) {
+    const bool in = kSpan * s + rq < rows;
+    const T* p = base(s) + (in ? offq : 0) + k;
+    T v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = p[min(QrMma<T>::row(g, e), nb - 1)];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int j = QrMma<T>::row(g, e);
+      x[e] = in && j < nb ? -vpick(kSpan * s + rq, j, v[e]) : T(0);
+    }
+  };
+  if (KR != 4 && wide) {
+    // ---- 64 columns, C read for W = V^T C and again for C - V (T^T W)
+    T(*s_wide)[NB][kWideLd] = reinterpret_cast<T(*)[NB][kWideLd]>(step_smem);  // [kWaves]
+    auto load_wide = [&](int s, M4 (&c)[kWideTiles]) {
+      const T* p = base(s);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const T* r = p + (exists(s, e) ? off[e] : 0);
+#pragma unroll
+        for (int u = 0; u < kWideTiles; ++u) c[u][e] = r[min(c0 + 16 * u + q, n - 1)];
+      }
+    };
+    M4 w[kWideTiles];
+#pragma unroll
+    for (int u = 0; u < kWideTiles; ++u) w[u] = M4{T(0), T(0), T(0), T(0)};
+#pragma unroll 2
+    for (int s = 0; s < ns; ++s) {
+      M4 c[kWideTiles];
+      T x[4];
+      load_wide(s, c);
+      project_v(s, x);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int u = 0; u < kWideTiles; ++u) w[u] = QrMma<T>::mul(x[e], exists(s, e) ? c[u][e] : T(0), w[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < kWideTiles; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s_wide[wv][QrMma<T>::row(g, e)][16 * u + q] = w[u][e];
+    __syncthreads();
+    M4 tw[kWideTiles];
+#pragma unroll
+    for (int u = 0; u < kWideTiles; ++u) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        T x = T(0);
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) x += s_wide[i][QrMma<T>::row(g, e)][16 * u + q];
+        w[u][e] = x;
+      }
+      tw[u] = M4{T(0), T(0), T(0), T(0)};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tw[u] = QrMma<T>::mul(tt[e], w[u][e], tw[u]);
+    }
+#pragma unroll 2
+    for (int s = 0; s < ns; ++s) {
+      M4 c[kWideTiles];
+      T x[4];
+      load_wide(s, c);
+      expand_v(s, x);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int u = 0; u < kWideTiles; ++u) c[u] = QrMma<T>::mul(x[e], tw[u][e], c[u]);
+      T* p = base(s);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int u = 0; u < kWideTiles; ++u)
+          if (exists(s, e) && c0 + 16 * u + q < n) p[off[e] + c0 + 16 * u + q] = c[u][e];
+    }
+    return;
+  }
   auto load = [&](int s) {
     const T* p = base(s) + min(col, n - 1);
     M4 v;
@@ -419,32 +561,15 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
   };
   if constexpr (KR > 0) each([&](int s, M4& v) __attribute__((always_inline)) { v = load(s); });
 
-  if (mode != kStepPanel) {
+  if (KR > 0 && mode != kStepPanel) {
     // ---- W = V^T C
-    const T* Tp = tblk + d.t_offset + (int64_t)(k / NB) * NB * NB;
-    T tt[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) tt[e] = Tp[QrMma<T>::row(g, e) * NB + q];
-    const int vc = k + min(q, nb - 1);
-    auto project = [&](int s, const M4& c, M4 w) {
-      const T* p = base(s) + vc;
-      T v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = p[exists(s, e) ? off[e] : 0];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const T x = vpick(kSpan * s + rel[e], q, v[e]);
-        w = QrMma<T>::mul(exists(s, e) && q < nb ? x : T(0), c[e], w);
-      }
-      return w;
-    };
     M4 w = {T(0), T(0), T(0), T(0)};
-    if constexpr (KR > 0) {
-      each_read([&](int s, const M4& v) __attribute__((always_inline)) { w = project(s, v, w); });
-    } else {
-#pragma unroll 4
-      for (int s = 0; s < ns; ++s) w = project(s, load(s), w);
-    }
+    each_read([&](int s, const M4& c) __attribute__((always_inline)) {
+      T x[4];
+      project_v(s, x);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w = QrMma<T>::mul(x[e], c[e], w);
+    });
 #pragma unroll
     for (int e = 0; e < 4; ++e) s_w[wv][QrMma<T>::row(g, e)][q] = w[e];
     __syncthreads();
@@ -459,32 +584,16 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
     M4 tw = {T(0), T(0), T(0), T(0)};
 #pragma unroll
     for (int e = 0; e < 4; ++e) tw = QrMma<T>::mul(tt[e], w[e], tw);
-    const int rq = 16 * wv + q;  // V by rows: row q of the tile
-    const int64_t offq = (int64_t)rq * lda;
-    auto subtract = [&](int s, M4 c) {
-      const bool in = kSpan * s + rq < rows;
-      const T* p = base(s) + (in ? offq : 0) + k;
-      T v[4];
+    each([&](int s, M4& c) __attribute__((always_inline)) {
+      T x[4];
+      expand_v(s, x);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = p[min(QrMma<T>::row(g, e), nb - 1)];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int j = QrMma<T>::row(g, e);
-        const T x = vpick(kSpan * s + rq, j, v[e]);
-        c = QrMma<T>::mul(in && j < nb ? -x : T(0), tw[e], c);
-      }
-      return c;
-    };
-    if constexpr (KR > 0) {
-      each([&](int s, M4& v) __attribute__((always_inline)) { v = subtract(s, v); });
-    } else {
-#pragma unroll 4
-      for (int s = 0; s < ns; ++s) store(s, subtract(s, load(s)));
-    }
+      for (int e = 0; e < 4; ++e) c = QrMma<T>::mul(x[e], tw[e], c);
+    });
   }
   if constexpr (KR > 0) {
     const int kn = mode == kStepPanel ? k : k + NB;  // the panel to factor
-    if (mode == kStepUpdate || blk != 0 || kn >= kmax) {
+    if (blk != 0 || kn >= kmax) {
       each_read([&](int s, const M4& v) __attribute__((always_inline)) { store(s, v); });
       return;
     }
@@ -607,8 +716,11 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
 
 template <typename T, int KR, int KL>
 int launch_step(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int mode, int k, const int32_t* kcol,
-                int blocks, T* a, T* tau, T* tblk) {
-  const size_t smem = sizeof(T) * (size_t)KL * 4 * kPanelThreads;
+                int right, T* a, T* tau, T* tblk) {
+  const int blocks = step_blocks(KR, mode, right);
+  const size_t far_bytes = sizeof(T) * (size_t)KL * 4 * kPanelThreads;
+  const size_t wide_bytes = KR == 4 ? 0 : sizeof(T) * (size_t)kPanelWaves * 16 * kWideLd;
+  const size_t smem = std::max(far_bytes, wide_bytes);
   if (smem) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&qr_step_kernel<T, KR, KL>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
@@ -626,20 +738,21 @@ int launch_step(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int mode
   return LXA_OK;
 }
 
-// rows bounds m - k over the systems; blocks is the number of 16-column blocks.
+// rows bounds m - k and right the columns right of the panel over the systems.
 template <typename T>
 int step(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int mode, int k, const int32_t* kcol, int rows,
-         int blocks, T* a, T* tau, T* tblk) {
-  if (rows <= 512) return launch_step<T, 4, 0>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
-  if (rows <= 1024) return launch_step<T, 8, 0>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
-  if (rows <= 2048) return launch_step<T, 16, 0>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
+         int right, T* a, T* tau, T* tblk) {
+  if (mode == kStepUpdate) return launch_step<T, 0, 0>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
+  if (rows <= 512) return launch_step<T, 4, 0>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
+  if (rows <= 1024) return launch_step<T, 8, 0>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
+  if (rows <= 2048) return launch_step<T, 16, 0>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
   if constexpr (sizeof(T) == 4) {
-    if (rows <= kStepMaxRows) return launch_step<T, 24, 8>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
+    if (rows <= kStepMaxRows) return launch_step<T, 24, 8>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
   } else {
-    if (rows <= 3072) return launch_step<T, 16, 8>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
-    if (rows <= kStepMaxRows) return launch_step<T, 24, 8>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
+    if (rows <= 3072) return launch_step<T, 16, 8>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
+    if (rows <= kStepMaxRows) return launch_step<T, 24, 8>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
   }
-  return launch_step<T, 0, 0>(st, count, desc, mode, k, kcol, blocks, a, tau, tblk);
+  return set_error(LXA_EINVAL, "qr step: panel of %d rows", rows);  // panel_only and qr_steps see to that
 }
 
 // ---------------------------------------------------------------------------
@@ -1010,43 +1123,36 @@ size_t trsv_smem_bytes(int dtype) {
   return e * (((kTrsvMaxK + 1) & ~1) + kTrsvBlock * (kTrsvBlock + 1) + kBigWaves * kWave + kTrsvBlock);
 }
 
-// Panels at column k_all (kcol == nullptr) or kcol[s] for system s.  max_rows
-// bounds m - k over the systems that still have columns.
+// Panels at column k (kcol == nullptr) or kcol[s] + k of system s.  max_rows
+// bounds the panels' rows over the systems that still have columns.
 template <typename T>
-int panel_only(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int k_all, const int32_t* kcol, int max_rows,
-               T* a, T* tau, T* tblk) {
-  if (max_rows <= kStepMaxRows) return step<T>(st, count, desc, kStepPanel, k_all, kcol, max_rows, 1, a, tau, tblk);
-  qr_panel_kernel<T><<<dim3((unsigned)count), kPanelThreads, 0, st>>>(desc, k_all, kcol, a, tau, tblk);
+int panel_only(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int k, const int32_t* kcol, int max_rows, T* a,
+               T* tau, T* tblk) {
+  if (max_rows <= kStepMaxRows) return step<T>(st, count, desc, kStepPanel, k, kcol, max_rows, 0, a, tau, tblk);
+  qr_panel_kernel<T><<<dim3((unsigned)count), kPanelThreads, 0, st>>>(desc, k, kcol, a, tau, tblk);
   LXA_LAUNCH_CHECK("qr_panel_kernel");
   return LXA_OK;
 }
 
-// One panel step for every system: factor the panel, update the columns right
-// of it.  max_trail_cols bounds n - k - 1.
+// `steps` panel steps of every system from column 0 (kcol == nullptr) or
+// kcol[s] on: each factors a panel and updates the columns right of it.
+// max_rows bounds m - kcol and max_right the columns right of the first panel
+// (n - kcol - 1, as a last panel may have a single column).  The update of a
+// step factors the panel of the next one, so only the first panel has a
+// launch of its own.
 template <typename T>
-int qr_step_impl(hipStream_t st, int64_t count, const lxa_qr_desc* desc, const int32_t* kcol, int max_rows,
-                 int max_trail_cols, T* a, T* tau, T* tblk) {
-  if (int rc = panel_only<T>(st, count, desc, 0, kcol, max_rows, a, tau, tblk)) return rc;
-  if (max_trail_cols <= 0) return LXA_OK;
-  return step<T>(st, count, desc, kStepUpdate, 0, kcol, max_rows, (max_trail_cols + 15) / 16, a, tau, tblk);
-}
-
-template <typename T>
-int qr_factor_impl(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int max_m, int max_n, int max_k, T* a,
-                   T* tau, T* tblk) {
+int qr_steps(hipStream_t st, int64_t count, const lxa_qr_desc* desc, const int32_t* kcol, int steps, int max_rows,
+             int max_right, T* a, T* tau, T* tblk) {
   constexpr int NB = QrCfg<T>::NB;
-  if (int rc = panel_only<T>(st, count, desc, 0, nullptr, max_m, a, tau, tblk)) return rc;
-  for (int k = 0; k < max_k; k += NB) {
-    // columns right of the panel: past it by its width, 1..16 columns
-    const int right = max_n - k - 1;
-    if (right <= 0) break;
-    const int rows = max_m - k;
-    const bool ahead = rows <= kStepMaxRows;
-    if (int rc = step<T>(st, count, desc, ahead ? kStepLookahead : kStepUpdate, k, nullptr, rows, (right + 15) / 16, a,
-                         tau, tblk))
+  if (int rc = panel_only<T>(st, count, desc, 0, kcol, max_rows, a, tau, tblk)) return rc;
+  for (int j = 0; j < steps; ++j) {
+    const int k = NB * j, rows = max_rows - k, right = max_right - k;
+    if (rows <= 0 || right <= 0) break;
+    const bool more = j + 1 < steps && rows > NB, ahead = more && rows <= kStepMaxRows;
+    if (int rc = step<T>(st, count, desc, ahead ? kStepLookahead : kStepUpdate, k, kcol, rows, right, a, tau, tblk))
       return rc;
-    if (!ahead && k + NB < max_k) {
-      if (int rc = panel_only<T>(st, count, desc, k + NB, nullptr, rows - NB, a, tau, tblk)) return rc;
+    if (more && !ahead) {
+      if (int rc = panel_only<T>(st, count, desc, k + NB, kcol, rows - NB, a, tau, tblk)) return rc;
     }
   }
   return LXA_OK;
@@ -1082,26 +1188,33 @@ extern "C" int lxa_qr_factor(void* stream, int dtype, int64_t count, const lxa_q
   LXA_REQUIRE(a && tau && tblk && work, "a, tau, tblk and work must be non-NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == LXA_F32)
-    return qr_factor_impl<float>(st, count, desc, max_m, max_n, max_k, static_cast<float*>(a),
-                                 static_cast<float*>(tau), static_cast<float*>(tblk));
-  return qr_factor_impl<double>(st, count, desc, max_m, max_n, max_k, static_cast<double*>(a),
-                                static_cast<double*>(tau), static_cast<double*>(tblk));
+    return qr_steps<float>(st, count, desc, nullptr, (max_k + 15) / 16, max_m, max_n - 1, static_cast<float*>(a),
+                           static_cast<float*>(tau), static_cast<float*>(tblk));
+  return qr_steps<double>(st, count, desc, nullptr, (max_k + 15) / 16, max_m, max_n - 1, static_cast<double*>(a),
+                          static_cast<double*>(tau), static_cast<double*>(tblk));
 }
 
 extern "C" int lxa_qr_factor_step(void* stream, int dtype, int64_t count, const lxa_qr_desc* desc,
                                   const int32_t* kcol, int max_rows, int max_trail_cols, void* a, void* tau,
                                   void* tblk, void* work) {
+  return lxa_qr_factor_steps(stream, dtype, count, desc, kcol, 1, max_rows, max_trail_cols, a, tau, tblk, work);
+}
+
+extern "C" int lxa_qr_factor_steps(void* stream, int dtype, int64_t count, const lxa_qr_desc* desc,
+                                   const int32_t* kcol, int steps, int max_rows, int max_trail_cols, void* a,
+                                   void* tau, void* tblk, void* work) {
+  LXA_REQUIRE(steps >= 0, "steps must be >= 0");
   if (int rc = check_batch(dtype, count, desc)) return rc;
   LXA_REQUIRE(kcol != nullptr, "kcol must be non-NULL");
   LXA_REQUIRE(max_rows >= 0, "max_rows must be >= 0");
-  if (count == 0 || max_rows == 0) return LXA_OK;
+  if (count == 0 || max_rows == 0 || steps == 0) return LXA_OK;
   LXA_REQUIRE(a && tau && tblk && work, "a, tau, tblk and work must be non-NULL");
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == LXA_F32)
-    return qr_step_impl<float>(st, count, desc, kcol, max_rows, max_trail_cols, static_cast<float*>(a),
-                               static_cast<float*>(tau), static_cast<float*>(tblk));
-  return qr_step_impl<double>(st, count, desc, kcol, max_rows, max_trail_cols, static_cast<double*>(a),
-                              static_cast<double*>(tau), static_cast<double*>(tblk));
+    return qr_steps<float>(st, count, desc, kcol, steps, max_rows, max_trail_cols, static_cast<float*>(a),
+                           static_cast<float*>(tau), static_cast<float*>(tblk));
+  return qr_steps<double>(st, count, desc, kcol, steps, max_rows, max_trail_cols, static_cast<double*>(a),
+                          static_cast<double*>(tau), static_cast<double*>(tblk));
 }
 
 extern "C" int lxa_qr_apply(void* stream, int dtype, int64_t count, const lxa_qr_desc* desc, int max_m, int max_k,

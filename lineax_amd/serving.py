@@ -7,8 +7,8 @@ The chosen form (``SolveServer(form="chosen")``) runs in ticks:
 1. admission: arrived requests are admitted first-come first-served while
    their working memory fits in the HBM arena (``hbm_budget`` bytes; the
    operator, its factors, scratch and right-hand side are allocated there);
-2. ``panels_per_tick`` launches of ``lxa_qr_factor_step`` advance every
-   admitted QR system by that many 16-column panels, each at its own column,
+2. one ``lxa_qr_factor_steps`` call advances every admitted QR system by
+   ``panels_per_tick`` 16-column panels, each at its own column,
    so systems admitted in different ticks share the launches (continuous
    batching);
 3. systems whose factorisation completed, and requests that reuse a resident
@@ -598,10 +598,7 @@ class SolveServer:
                     # (descriptors, events, polling) is paid once for them;
                     # systems past their last column are skipped by the kernels
                     steps = min(self.panels_per_tick, -(-max(r.n - k for r, _, k in factoring) // self.nb))
-                    for j in range(steps):
-                        if j:
-                            kcol += self.nb
-                        K.qr_factor_step_raw(dd, len(factoring), kcol, max_rows, max_tc, buf, buf, buf, buf)
+                    K.qr_factor_step_raw(dd, len(factoring), kcol, max_rows, max_tc, buf, buf, buf, buf, steps)
                     nxt = []
                     for f in factoring:
                         f[2] += self.nb * steps
