@@ -747,9 +747,9 @@ int step(hipStream_t st, int64_t count, const lxa_qr_desc* desc, int mode, int k
   if (rows <= 1024) return launch_step<T, 8, 0>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
   if (rows <= 2048) return launch_step<T, 16, 0>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
   if constexpr (sizeof(T) == 4) {
-    if (rows <= kStepMaxRows) return launch_step<T, 24, 8>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
+    if (rows <= kStepMaxRows) return launch_step<T, 28, 4>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
   } else {
-    if (rows <= 3072) return launch_step<T, 16, 8>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
+    if (rows <= 3072) return launch_step<T, 20, 4>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
     if (rows <= kStepMaxRows) return launch_step<T, 24, 8>(st, count, desc, mode, k, kcol, right, a, tau, tblk);
   }
   return set_error(LXA_EINVAL, "qr step: panel of %d rows", rows);  // panel_only and qr_steps see to that
@@ -829,21 +829,47 @@ __global__ __launch_bounds__(kBigThreads) void qr_apply_kernel(const lxa_qr_desc
 // RPT panel entries in registers between the reduction and the update (V is
 // read once per panel); RPT == 0 reads them twice.  Per panel:
 //   w = V^T x (lanes of a column, then waves, summed in a fixed order);
-//   w = T^T w or T w (wave 0, shuffles);  x -= V w (NB-lane row sums).
+//   w = T^T w or T w (wave 0, shuffles);  x -= V w (row sums of up to 16 rows
+//   at a time by a reduce-scatter over their 16 lanes).
+// One double system of 3001 x 391, its panels read twice in rounds of eight
+// rows and a four-step butterfly per row: 763 us.
 // ---------------------------------------------------------------------------
 constexpr int kApplyMaxRows = 16384;
 
-template <typename T, int RPT>
-__global__ __launch_bounds__(kBigThreads) void qr_apply_rows_kernel(const lxa_qr_desc* __restrict__ descs,
+// Sums K values (K a power of two <= 16) over the 16 lanes of a row; lane j
+// of the row holds the sum of value j / (16 / K).  v is destroyed.
+template <int K, int L = 0, typename T>
+__device__ __forceinline__ T row_reduce_scatter(T (&v)[K], int j) {
+  constexpr int off = 8 >> L, half = K >> (L + 1);
+  if constexpr (off == 0) {
+    return v[0];
+  } else if constexpr (half >= 1) {
+    const bool upper = (j & off) != 0;
+#pragma unroll
+    for (int i = 0; i < half; ++i) {
+      const T keep = upper ? v[i + half] : v[i];
+      const T send = upper ? v[i] : v[i + half];
+      v[i] = keep + lane_xor<off>(send);
+    }
+    return row_reduce_scatter<K, L + 1>(v, j);
+  } else {
+    v[0] += lane_xor<off>(v[0]);
+    return row_reduce_scatter<K, L + 1>(v, j);
+  }
+}
+
+template <typename T, int RPT, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void qr_apply_rows_kernel(const lxa_qr_desc* __restrict__ descs,
                                                                       const T* __restrict__ a,
                                                                       const T* __restrict__ tblk,
                                                                       T* __restrict__ b, int trans) {
   constexpr int NB = QrCfg<T>::NB;
   constexpr int G = kWave / NB;       // rows per wave load
-  constexpr int RP = kBigWaves * G;   // rows per pass of the workgroup
+  constexpr int RP = WAVES * G;       // rows per pass of the workgroup
+  constexpr int kBlock = WAVES * kWave;
   extern __shared__ __align__(16) unsigned char apply_smem[];
   T* xs = reinterpret_cast<T*>(apply_smem);
-  __shared__ T s_part[kBigWaves][NB];
+  __shared__ T s_part[WAVES][NB];
   __shared__ T s_w[NB];
   const lxa_qr_desc d = descs[blockIdx.x];
   const int m = d.m, lda = d.lda;
@@ -853,7 +879,7 @@ __global__ __launch_bounds__(kBigThreads) void qr_apply_rows_kernel(const lxa_qr
   const int j = lane % NB, rg = wv * G + lane / NB;
   const T* A = a + d.a_offset;
   T* x = b + d.b_offset + (int64_t)blockIdx.y * d.ldb;
-  for (int i = tid; i < m; i += kBigThreads) xs[i] = x[i];
+  for (int i = tid; i < m; i += kBlock) xs[i] = x[i];
   __syncthreads();
   const int panels = (kmax + NB - 1) / NB;
   T v[RPT > 0 ? RPT : 1];
@@ -879,6 +905,7 @@ __global__ __launch_bounds__(kBigThreads) void qr_apply_rows_kernel(const lxa_qr
         const int row = k + rg + t * RP;
         const T st = Ak[(int64_t)min(row, m - 1) * lda];
         v[t] = (row < m && j < nb) ? vpick(row, k + j, st) : T(0);
+        if (t % 16 == 15) __builtin_amdgcn_sched_barrier(0);  // addresses of 16 rows at a time
       }
 #pragma unroll
       for (int t = 0; t < RPT; ++t) {
@@ -906,7 +933,7 @@ __global__ __launch_bounds__(kBigThreads) void qr_apply_rows_kernel(const lxa_qr
       T wsum = T(0);
       if (lane < NB) {
 #pragma unroll
-        for (int w = 0; w < kBigWaves; ++w) wsum += s_part[w][lane];
+        for (int w = 0; w < WAVES; ++w) wsum += s_part[w][lane];
       }
       T s = T(0);
 #pragma unroll
@@ -925,13 +952,15 @@ __global__ __launch_bounds__(kBigThreads) void qr_apply_rows_kernel(const lxa_qr
     __syncthreads();
     const T wj = s_w[j];
     if constexpr (RPT > 0) {
+      constexpr int K = RPT < NB ? RPT : NB;
 #pragma unroll
-      for (int t = 0; t < RPT; ++t) {
-        const int row = k + rg + t * RP;
-        T s = v[t] * wj;
+      for (int t0 = 0; t0 < RPT; t0 += K) {
+        T s[K];
 #pragma unroll
-        for (int off = 1; off < NB; off <<= 1) s += __shfl_xor(s, off, kWave);
-        if (j == 0 && row < m) xs[row] -= s;
+        for (int t = 0; t < K; ++t) s[t] = v[t0 + t] * wj;
+        const T sum = row_reduce_scatter<K>(s, j);
+        const int row = k + rg + (t0 + j / (NB / K)) * RP;
+        if (j % (NB / K) == 0 && row < m) xs[row] -= sum;
       }
     } else {
       for (int row0 = k + rg; row0 < m; row0 += 8 * RP) {
@@ -950,19 +979,18 @@ __global__ __launch_bounds__(kBigThreads) void qr_apply_rows_kernel(const lxa_qr
     }
     __syncthreads();
   }
-  for (int i = tid; i < m; i += kBigThreads) x[i] = xs[i];
+  for (int i = tid; i < m; i += kBlock) x[i] = xs[i];
 }
 
-template <typename T, int RPT>
+template <typename T, int RPT, int WAVES>
 int launch_apply_rows(hipStream_t st, dim3 grid, int max_m, const lxa_qr_desc* desc, const void* a, const void* tblk,
                       void* b, int trans) {
   const size_t smem = sizeof(T) * (size_t)max_m;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&qr_apply_rows_kernel<T, RPT>),
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&qr_apply_rows_kernel<T, RPT, WAVES>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (e != hipSuccess) return hip_error(e, "hipFuncSetAttribute(qr_apply_rows)");
-  qr_apply_rows_kernel<T, RPT><<<grid, kBigThreads, smem, st>>>(desc, static_cast<const T*>(a),
-                                                                 static_cast<const T*>(tblk), static_cast<T*>(b),
-                                                                 trans);
+  qr_apply_rows_kernel<T, RPT, WAVES><<<grid, WAVES * kWave, smem, st>>>(
+      desc, static_cast<const T*>(a), static_cast<const T*>(tblk), static_cast<T*>(b), trans);
   LXA_LAUNCH_CHECK("qr_apply_rows_kernel");
   return LXA_OK;
 }
@@ -970,14 +998,16 @@ int launch_apply_rows(hipStream_t st, dim3 grid, int max_m, const lxa_qr_desc* d
 template <typename T>
 int apply_rows(hipStream_t st, dim3 grid, int max_m, const lxa_qr_desc* desc, const void* a, const void* tblk,
                void* b, int trans) {
-  constexpr int RP = kBigWaves * (kWave / QrCfg<T>::NB);
-  constexpr int kMaxRpt = sizeof(T) == 4 ? 32 : 16;  // no spills under the 128-VGPR cap of 1024 threads
-  const int rpt = (max_m + RP - 1) / RP;
-  if (rpt <= 4) return launch_apply_rows<T, 4>(st, grid, max_m, desc, a, tblk, b, trans);
-  if (rpt <= 8) return launch_apply_rows<T, 8>(st, grid, max_m, desc, a, tblk, b, trans);
-  if (rpt <= 16) return launch_apply_rows<T, 16>(st, grid, max_m, desc, a, tblk, b, trans);
-  if (rpt <= kMaxRpt) return launch_apply_rows<T, kMaxRpt>(st, grid, max_m, desc, a, tblk, b, trans);
-  return launch_apply_rows<T, 0>(st, grid, max_m, desc, a, tblk, b, trans);
+  // 16 waves up to 16 panel entries per lane (128 registers each), then eight
+  // waves, which have 256: up to 2048 rows, then as many as they hold
+  constexpr int kPass = kWave / QrCfg<T>::NB;  // rows per wave load
+  constexpr int kMost = sizeof(T) == 4 ? 128 : 96;
+  if (max_m <= 4 * 16 * kPass) return launch_apply_rows<T, 4, 16>(st, grid, max_m, desc, a, tblk, b, trans);
+  if (max_m <= 8 * 16 * kPass) return launch_apply_rows<T, 8, 16>(st, grid, max_m, desc, a, tblk, b, trans);
+  if (max_m <= 16 * 16 * kPass) return launch_apply_rows<T, 16, 16>(st, grid, max_m, desc, a, tblk, b, trans);
+  if (max_m <= 64 * 8 * kPass) return launch_apply_rows<T, 64, 8>(st, grid, max_m, desc, a, tblk, b, trans);
+  if (max_m <= kMost * 8 * kPass) return launch_apply_rows<T, kMost, 8>(st, grid, max_m, desc, a, tblk, b, trans);
+  return launch_apply_rows<T, 0, 16>(st, grid, max_m, desc, a, tblk, b, trans);
 }
 
 // ---------------------------------------------------------------------------
