@@ -120,6 +120,9 @@ class AbstractLinearSolver(abc.ABC):
 
 
 def _result_tensor(result, batch: tuple, device) -> torch.Tensor:
+    if not isinstance(result, torch.Tensor):
+        # filled on the device: a copy from the host would wait for the stream
+        return torch.full(batch, int(result), dtype=torch.int32, device=device)
     r = torch.as_tensor(result, dtype=torch.int32, device=device)
     return r.expand(batch).contiguous().clone() if r.shape != tuple(batch) else r.contiguous().clone()
 
@@ -144,8 +147,8 @@ def _linear_solve_impl(operator, state, vector, options, solver, throw: bool):
         else:
             K.solve_results(flat_s, flat_v.to(flat_s.dtype), result)
     if throw:
-        bad = result != RESULTS.successful
-        if bool(bad.any()):
+        # codes other than successful (0) are not zero; one code is read as it is
+        if bool(result) if result.dim() == 0 else bool(result.any()):
             raise RuntimeError(RESULTS[result])
     return solution, result, stats
 
