@@ -179,13 +179,7 @@ __device__ __forceinline__ int packed_upper(int n, int i, int j) {
   return i * n - ((i * (i - 1)) >> 1) + (j - i);
 }
 
-// Register-tiled Cholesky factor of a uniform float32 batch, orders 1..256
-// (chol_uneven.hip); same layout, NaN-on-failure and info conventions as
-// lxa_chol_factor.
-int chol_factor_regs_f32(hipStream_t s, int64_t batch, int n, float* a, int64_t stride, int negate, int32_t* info);
-
-// Cholesky factor and solve of orders past the one-workgroup tiers
-// (chol_tiled.hip); conventions of lxa_chol_factor / lxa_chol_solve.
+// Cholesky factor and solve in tiles (chol_tiled.hip); conventions of lxa_chol_factor / lxa_chol_solve.
 int chol_tile_factor(hipStream_t s, int64_t batch, int n, float* a, int64_t stride, int negate, int32_t* info);
 int chol_tile_factor(hipStream_t s, int64_t batch, int n, double* a, int64_t stride, int negate, int32_t* info);
 int chol_tile_solve(hipStream_t s, int64_t batch, int n, const float* u, int64_t us, float* b, int64_t bs, int negate);
