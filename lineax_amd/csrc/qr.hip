@@ -136,7 +136,18 @@ __global__ __launch_bounds__(kPanelThreads) void qr_panel_kernel(const lxa_qr_de
   const int tid = threadIdx.x;
   T* A = a + d.a_offset;
   const int nr = (m - k + kPanelThreads - 1) / kPanelThreads;
-  auto P = [&](int r, int c) -> T& { return A[(int64_t)(k + tid + r * kPanelThreads) * lda + k + c]; };
+  // a row's panel entries, all loads unconditional where the panel is whole
+  // (a test per column had made each wait for the one before)
+  auto load_row = [&](int row, T (&v)[NB]) {
+    const T* p = A + (int64_t)row * lda + k;
+    if (nb == NB) {
+#pragma unroll
+      for (int c = 0; c < NB; ++c) v[c] = p[c];
+    } else {
+#pragma unroll
+      for (int c = 0; c < NB; ++c) v[c] = c < nb ? p[c] : T(0);
+    }
+  };
 
   T taus[NB];
   // the column loop at compile time (every register index a constant)
@@ -157,19 +168,20 @@ __global__ __launch_bounds__(kPanelThreads) void qr_panel_kernel(const lxa_qr_de
     T dots[KW];
 #pragma unroll
     for (int c = 0; c < KW; ++c) dots[c] = T(0);
+#pragma unroll 2
     for (int r = 0; r < nr; ++r) {
       const int row = k + tid + r * kPanelThreads;
-      if (row < m && row > diag) {
-        const T x = P(r, j);
-        nv[0] += (double)x * (double)x;
+      T v[NB];
+      load_row(min(row, m - 1), v);
+      const T x = row < m && row > diag ? v[j] : T(0);
+      nv[0] += (double)x * (double)x;
 #pragma unroll
-        for (int c = 0; c < NB; ++c)
-          if (c != j && c < nb) dots[c] += x * P(r, c);
-      }
+      for (int c = 0; c < NB; ++c)
+        if (c != j) dots[c] += x * v[c];
     }
     if (tid == j) {
 #pragma unroll
-      for (int c = 0; c < NB; ++c) sd[c] = c < nb ? P(0, c) : T(0);
+      for (int c = 0; c < NB; ++c) sd[c] = c < nb ? A[(int64_t)diag * lda + k + c] : T(0);
     }
     block_sum2<1, KW, kPanelWaves>(nv, s_stage2, s_out2, dots, s_stage, s_out, tid);
     const double ss = nv[0], alpha = (double)sd[j];
@@ -194,18 +206,25 @@ __global__ __launch_bounds__(kPanelThreads) void qr_panel_kernel(const lxa_qr_de
     for (int r = 0; r < nr; ++r) {
       const int row = k + tid + r * kPanelThreads;
       if (row < m && row >= diag) {
-        T vj = T(1);
-        if (row > diag) {
-          vj = P(r, j) * scale;
-          if (ss != 0.0) P(r, j) = vj;
-        } else {
-          P(r, j) = beta;
+        T v[NB];
+        load_row(row, v);
+        T* p = A + (int64_t)row * lda + k;
+        const T vj = row > diag ? v[j] * scale : T(1);
+        if (row == diag) {
+          p[j] = beta;
+        } else if (ss != 0.0) {
+          p[j] = vj;
         }
         if (tj != T(0)) {
           const T tv = tj * vj;
+          if (nb == NB) {
 #pragma unroll
-          for (int c = 0; c < NB; ++c)
-            if (c > j && c < nb) P(r, c) -= tv * acc[c];
+            for (int c = j + 1; c < NB; ++c) p[c] = v[c] - tv * acc[c];
+          } else {
+#pragma unroll
+            for (int c = j + 1; c < NB; ++c)
+              if (c < nb) p[c] = v[c] - tv * acc[c];
+          }
         }
       }
     }
