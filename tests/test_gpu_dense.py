@@ -183,8 +183,7 @@ def test_cholesky_matches_oracle(device, rng, n, dtype):
 @pytest.mark.parametrize("n", [6, 70, 200, 300])
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 def test_cholesky_failure_is_singular(device, rng, n, dtype):
-    # float32 orders 65..256 take the register-tiled factor, the rest the
-    # lane-per-row, LDS and global-memory tiers
+    # orders above 64 take the tiled factor, the rest the lane-per-row tier
     a = well_conditioned(rng, n, kind="psd")
     a[n // 2, n // 2] = -5.0
     op = lx.MatrixLinearOperator(_t(a, device, dtype), lx.positive_semidefinite_tag)
