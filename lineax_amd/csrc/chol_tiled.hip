@@ -303,14 +303,14 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 2) void chol_tile_ke
     const int others = 16 * ctiles - r0 - kS;
     const int oc = wv * 48 + lane - kS;
     const int col = lane < kS ? r0 + lane : r0 + kS + min(oc, others - 1);
-    const bool mine = lane < kS ? wv == 0 : oc < others;
+    const bool diag = wv == 0 && lane < kS;  // wave 0 keeps the factored block, the others work on copies
+    T* Ms = M + r0 * kLd + (others > 0 ? col : min(col, r0 + kS - 1));
+    T c[kS];
     if (wv == 0 || wv * 48 < others) {  // uniform
       // opaque per strip: the 16 lane masks are formed where they are used
       // instead of being held, and spilled, across the strips
       int ln = lane;
       asm volatile("" : "+v"(ln));
-      T c[kS];
-      T* Ms = M + r0 * kLd + (others > 0 ? col : min(col, r0 + kS - 1));
 #pragma unroll
       for (int i = 0; i < kS; ++i) c[i] = Ms[i * kLd];
       unroll<0, kS>([&](auto T_) __attribute__((always_inline)) {
@@ -330,12 +330,18 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 2) void chol_tile_ke
           c[i] -= from_lane(c[p], i) * c[p];
         });
       });
-      if (mine) {
+      if (lane >= kS && oc < others) {
 #pragma unroll
         for (int i = 0; i < kS; ++i) Ms[i * kLd] = c[i];
       }
     }
     __syncthreads();
+    // the factored diagonal block goes over the one that every wave has read
+    // above, so behind the barrier; the update below takes no column of it
+    if (diag) {
+#pragma unroll
+      for (int i = 0; i < kS; ++i) Ms[i * kLd] = c[i];
+    }
     // ---- the rows below: M_rc -= M_sr^T M_sc, 16 x 16 tiles dealt to the
     // waves (row strip r, column tile c >= r)
     int idx = wv;

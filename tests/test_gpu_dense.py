@@ -262,6 +262,21 @@ def test_cholesky_tiled(device, rng, n, dtype):
         assert bool((r.abs() <= 2 * (3 * n + 2) * eps * scale).all())
 
 
+@pytest.mark.parametrize("n,dtype", [(80, torch.float32), (200, torch.float32), (256, torch.float32),
+                                     (100, torch.float64), (150, torch.float64), (257, torch.float64)])
+def test_cholesky_tiled_copies_agree(device, rng, n, dtype):
+    """Copies of one system, several workgroups to a compute unit, give the bits
+    that the system gives alone: the four waves of a panel tile read each strip's
+    diagonal block, and none may meet the block that one of them has factored."""
+    a = _t(well_conditioned(rng, n, kind="psd"), device, dtype)
+    alone, info = K.chol_factor(a[None])
+    assert info.tolist() == [0]
+    for _ in range(3):
+        u, info = K.chol_factor(a.expand(700, n, n).contiguous())
+        assert not bool(info.any())
+        assert torch.equal(u, alone.expand_as(u))
+
+
 def test_gemv_matches(device, rng):
     # (5000, 300) and (4099, 37) split the transposed product over row chunks
     # (the 16-byte path and the scalar path); the rest run in one chunk
