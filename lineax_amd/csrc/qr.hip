@@ -136,8 +136,9 @@ __global__ __launch_bounds__(kPanelThreads) void qr_panel_kernel(const lxa_qr_de
   const lxa_qr_desc d = descs[blockIdx.x];
   const int m = d.m, n = d.n, lda = d.lda;
   const int kmax = min(m, n);
-  const int k = (kcol ? kcol[blockIdx.x] : 0) + k_all;
-  if (k >= kmax) return;
+  const int kc = kcol ? kcol[blockIdx.x] : 0;
+  if (kc >= kmax - k_all) return;  // no sum here: a system that is done may say so by any large column
+  const int k = kc + k_all;
   const int nb = min(NB, kmax - k);
   const int tid = threadIdx.x;
   T* A = a + d.a_offset;
@@ -414,8 +415,9 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
   const lxa_qr_desc d = descs[sys];
   const int m = d.m, n = d.n, lda = d.lda;
   const int kmax = min(m, n);
-  const int k = (kcol ? kcol[sys] : 0) + k_all;
-  if (k >= kmax) return;
+  const int kc = kcol ? kcol[sys] : 0;
+  if (kc >= kmax - k_all) return;  // no sum here: a system that is done may say so by any large column
+  const int k = kc + k_all;
   const int nb = min(NB, kmax - k);
   const bool wide = mode == kStepUpdate || (mode == kStepLookahead && KR > 4 && blk > 0);
   const int c0 = mode == kStepPanel      ? k

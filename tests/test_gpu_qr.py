@@ -65,17 +65,34 @@ def test_geqrf_f32_close_to_f64(device, rng, shape):
     assert np.max(np.abs(r_got - r_ref)) <= tol * np.max(np.abs(r_ref))
 
 
+def _check_factor(exact, h, tau, tblk, u):
+    """Column j of A - Q R is below m n u |a_j| and Q^T Q - I below m n u
+    (Higham, Accuracy and Stability, thm 19.4 with c = 1), the compact-WY blocks
+    to the same; everything in double but made with unit roundoff u."""
+    m, n = exact.shape
+    k, nb = min(m, n), tblk.shape[-1]
+    v = np.tril(h[:, :k], -1) + np.eye(m, k)
+    q = np.eye(m, k)
+    for j in reversed(range(k)):
+        q -= tau[j] * np.outer(v[:, j], v[:, j] @ q)
+    r = np.triu(h[:k])
+    err = np.linalg.norm(exact - q @ r, axis=0)
+    assert np.all(err <= m * n * u * np.linalg.norm(exact, axis=0))
+    assert np.linalg.norm(q.T @ q - np.eye(k), 2) <= m * n * u
+    wy = np.eye(m, k)
+    for p in reversed(range(tblk.shape[0])):
+        vp = v[:, p * nb: p * nb + nb]
+        wy -= vp @ (tblk[p][: vp.shape[1], : vp.shape[1]] @ (vp.T @ wy))
+    assert np.linalg.norm(wy - q, 2) <= m * n * u
+
+
 @pytest.mark.parametrize("shape", [(15, 15), (512, 33), (513, 33), (528, 17), (1025, 40), (2049, 31), (2064, 40),
                                    (3073, 20), (3100, 50), (4096, 18), (4097, 18), (4112, 33), (18, 530), (40, 71)])
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 def test_geqrf_step_edges(device, rng, shape, dtype):
     """Heights around the step kernel's tiles and register / LDS limits, widths
     that leave partial panels, wide matrices, three systems with one of them
-    rank deficient.
-
-    Bounds: column j of A - Q R is below m n u |a_j| and Q^T Q - I below m n u
-    (Higham, Accuracy and Stability, thm 19.4 with c = 1), the compact-WY blocks
-    to the same."""
+    rank deficient; bounds in _check_factor."""
     m, n = shape
     k = min(m, n)
     u = torch.finfo(dtype).eps / 2
@@ -87,21 +104,53 @@ def test_geqrf_step_edges(device, rng, shape, dtype):
     exact = t.cpu().double().numpy()
     h, tau, tblk = ad.cpu().double().numpy(), tau.cpu().double().numpy(), tblk.cpu().double().numpy()
     assert tau[2, k // 2] == 0.0 or np.abs(h[2, k // 2:, k // 2]).max() < 1.0
-    nb = tblk.shape[-1]
     for i in range(3):
-        v = np.tril(h[i][:, :k], -1) + np.eye(m, k)
-        q = np.eye(m, k)
-        for j in reversed(range(k)):
-            q -= tau[i, j] * np.outer(v[:, j], v[:, j] @ q)
-        r = np.triu(h[i][:k])
-        err = np.linalg.norm(exact[i] - q @ r, axis=0)
-        assert np.all(err <= m * n * u * np.linalg.norm(exact[i], axis=0))
-        assert np.linalg.norm(q.T @ q - np.eye(k), 2) <= m * n * u
-        wy = np.eye(m, k)
-        for p in reversed(range(tblk.shape[1])):
-            vp = v[:, p * nb: p * nb + nb]
-            wy -= vp @ (tblk[i, p][: vp.shape[1], : vp.shape[1]] @ (vp.T @ wy))
-        assert np.linalg.norm(wy - q, 2) <= m * n * u
+        _check_factor(exact[i], h[i], tau[i], tblk[i], u)
+
+
+@pytest.mark.parametrize("steps", [2, 3, 6])
+@pytest.mark.parametrize("shapes", [[(400, 90), (512, 130), (100, 200), (40, 33)],
+                                    [(700, 300), (300, 200), (2100, 70), (33, 33)],
+                                    [(4200, 40), (900, 100), (20, 7)]])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_qr_factor_steps_from_own_columns(device, rng, dtype, shapes, steps):
+    """Several panel steps a call, every system at its own column: systems that
+    start late, finish inside a call, or are done (any column past the last,
+    the largest integer too), panels of up to 512 rows and above, above 4096;
+    bounds in _check_factor."""
+    nb, done = K.qr_block(dtype), 2**31 - 1
+    mats = [_t(rng.standard_normal(s), device, dtype) for s in shapes]
+    descs = np.zeros(len(shapes), dtype=K.QR_DESC)
+    a_off = tau_off = t_off = 0
+    for i, (m, n) in enumerate(shapes):
+        k = min(m, n)
+        descs[i] = (a_off, tau_off, t_off, 0, 0, m, n, n, 0)
+        a_off, tau_off, t_off = a_off + m * n, tau_off + k, t_off + -(-k // nb) * nb * nb
+    a = torch.cat([x.reshape(-1) for x in mats])
+    tau = torch.zeros(tau_off, dtype=dtype, device=device)
+    tblk = torch.zeros(t_off, dtype=dtype, device=device)
+    dd = K.descs_to_device(descs, device)
+    cols, call = [0] * len(shapes), 0
+    while any(c < min(s) for c, s in zip(cols, shapes)):
+        live = [i for i, s in enumerate(shapes) if i <= call and cols[i] < min(s)]  # system i joins at call i
+        if live:
+            at = [c if i in live else done for i, c in enumerate(cols)]
+            K.qr_factor_step_raw(dd, len(shapes), torch.tensor(at, dtype=torch.int32).to(device),
+                                 max(shapes[i][0] - cols[i] for i in live),
+                                 max(shapes[i][1] - cols[i] - 1 for i in live), a, tau, tblk, tau, steps)
+        for i in live:
+            cols[i] += nb * steps
+        call += 1
+    u = torch.finfo(dtype).eps / 2
+    for i, (m, n) in enumerate(shapes):
+        k = min(m, n)
+        panels = -(-k // nb)
+        d = {name: int(descs[i][name]) for name in ("a_offset", "tau_offset", "t_offset")}
+        _check_factor(mats[i].cpu().double().numpy(),
+                      a[d["a_offset"]: d["a_offset"] + m * n].cpu().double().numpy().reshape(m, n),
+                      tau[d["tau_offset"]: d["tau_offset"] + k].cpu().double().numpy(),
+                      tblk[d["t_offset"]: d["t_offset"] + panels * nb * nb].cpu().double().numpy()
+                      .reshape(panels, nb, nb), u)
 
 
 def test_geqrf_zero_column_gives_zero_tau(device):
