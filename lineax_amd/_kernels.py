@@ -892,6 +892,11 @@ def qr_solve(a: torch.Tensor, tblk: torch.Tensor, b: torch.Tensor, transpose: bo
     op_lead = tuple(a.shape[:-2])
     lead = tuple(torch.broadcast_shapes(op_lead, b.shape[:-1]))
     nb = qr_block(a.dtype)
+    # the kernels address T blocks of this width: others (a factor saved when
+    # float64 panels had 8 columns) would be read past their end
+    if tuple(tblk.shape) != (*op_lead, -(-N // nb), nb, nb):
+        raise ValueError(f"T blocks of shape {tuple(tblk.shape)} do not belong to a {tuple(a.shape)} factor in "
+                         f"panels of {nb} columns: factor the matrix again")
     descs, count = _solve_descs(lead, op_lead, M, N, nb, M, a.device)
     buf = torch.zeros((*lead, M), dtype=a.dtype, device=a.device)
     if count == 0:

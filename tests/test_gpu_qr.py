@@ -221,6 +221,17 @@ def test_qr_transpose_state_reuse(device, rng):
     np.testing.assert_allclose(x_t.cpu().numpy(), np.linalg.lstsq(a.T, c, rcond=None)[0], rtol=1e-10, atol=1e-10)
 
 
+def test_qr_solve_refuses_other_t_blocks(device, rng):
+    """T blocks that are not the factor's (8-wide ones, of another order or
+    batch) are an error on the host, not reads past their end."""
+    b = _t(rng.standard_normal((2, 40)), device)
+    a, tau, tblk = K.qr_factor(_t(rng.standard_normal((2, 40, 25)), device))
+    for bad in (torch.zeros(2, 4, 8, 8, dtype=b.dtype, device=device), tblk[:, :1], tblk[:1]):
+        with pytest.raises(ValueError, match="factor the matrix again"):
+            K.qr_solve(a, bad, b, False)
+    assert bool(torch.isfinite(K.qr_solve(a, tblk, b, False)).all())
+
+
 def test_qr_grad_square_closed_form(device, rng):
     a = rng.standard_normal((12, 12)) + 4 * np.eye(12)
     b = rng.standard_normal(12)
