@@ -361,6 +361,19 @@ __device__ __forceinline__ void reflector(double alpha, double ss, double& beta,
   }
 }
 
+// Whether v_q^T v_j may be formed as scales of v_q and v_j times a sum over the
+// unscaled columns (larft in qr_step_kernel): the sum's products, of which
+// there are at most 2^12 with norms below 1 / |sq| and 1 / |sj|, neither
+// overflow nor lose more than rounding to the smallest normal number.
+__device__ __forceinline__ bool unscaled_sums(float sq, float sj) {
+  const float p = fabsf(sq * sj);
+  return p >= 0x1p-100f && p <= 0x1p80f && fabsf(sq) <= 0x1p100f;
+}
+__device__ __forceinline__ bool unscaled_sums(double sq, double sj) {
+  const double p = fabs(sq * sj);
+  return p >= 0x1p-960 && p <= 0x1p900 && fabs(sq) <= 0x1p960;
+}
+
 // What a launch does with the panel at column k.
 enum : int {
   kStepPanel = 0,      // factor it (one workgroup per system)
@@ -629,6 +642,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
     const int nbn = min(NB, kmax - kn);
     const int t0 = (kn - k) / 16;  // tile with the panel's diagonal: slot 0 of wave t0
     T sc = T(1);                   // scaling of this lane's column below its diagonal, applied when stored
+    bool rescale = false;          // products of this lane's column with a later one are out of range
     static_for<0, NB>([&](auto J_) __attribute__((always_inline)) {
       constexpr int j = decltype(J_)::value;
       if (j >= nbn) return;  // uniform
@@ -681,6 +695,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
       }
       // v = [1; scale x]: v^T (column q) for q > j (larf), v_q^T v for q < j
       // (larft; columns left of j are still unscaled)
+      rescale = rescale || (ss != 0.0 && q < j && !unscaled_sums(sc, scale));
       const T prod = dv + scale * dots;
       if (tid < j) s_g[tid][j] = sc * prod;
       if (tid == j) s_tau[j] = tj;
@@ -704,15 +719,36 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
         for (int e = 0; e < 4; ++e) v[e] = fma(row_bcast<j>(v[e]), coef, v[e]);
       });
     });
-    each_read([&](int s, const M4& v) __attribute__((always_inline)) {
-      M4 o;
+    // column q of V from here on, with R above it
+    each([&](int s, M4& v) __attribute__((always_inline)) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const bool below = s > 0 || wv > t0 || (wv == t0 && QrMma<T>::row(g, e) > q);
-        o[e] = below ? v[e] * sc : v[e];
+        v[e] = below ? v[e] * sc : v[e];
       }
-      store(s, o);
+      store(s, v);
     });
+    if (__any(rescale)) {  // uniform over the workgroup: every wave holds all columns' scales
+      // ---- V^T V from the scaled columns: a result register is both operands
+      M4 w = {T(0), T(0), T(0), T(0)};
+      each_read([&](int s, const M4& v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = kSpan * s + rel[e] - 16 * t0;
+          const T x = q < nbn ? vpick(r, q, v[e]) : T(0);
+          w = QrMma<T>::mul(x, x, w);
+        }
+      });
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s_w[wv][QrMma<T>::row(g, e)][q] = w[e];
+      __syncthreads();
+      if (tid < NB * NB) {
+        T x = T(0);
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) x += s_w[i][tid / NB][tid % NB];
+        s_g[tid / NB][tid % NB] = x;
+      }
+    }
     __syncthreads();  // s_g and s_tau complete
 
     // ---- T (larft, forward, columnwise): lane a owns row a of T.

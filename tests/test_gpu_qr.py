@@ -108,6 +108,41 @@ def test_geqrf_step_edges(device, rng, shape, dtype):
         _check_factor(exact[i], h[i], tau[i], tblk[i], u)
 
 
+@pytest.mark.parametrize("shape", [(200, 16), (500, 40), (700, 23), (1500, 20), (2500, 20), (3300, 20), (4000, 20),
+                                   (4200, 20)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_geqrf_t_blocks_of_small_columns(device, rng, shape, dtype):
+    """Columns whose products underflow, or would overflow where the reflectors'
+    do not: nearly dependent ones of small and of large scale, small ones beside
+    others, equal ones.  I - V T V^T is the product of the reflectors as for any
+    data: m n u bounds their difference (_check_factor); all of the factor is
+    checked where its own norms and products stay in range."""
+    m, n = shape
+    tiny = 1e-17 if dtype == torch.float32 else 1e-150
+    u = torch.finfo(dtype).eps / 2
+    base = rng.standard_normal((m, n))
+    near = base[:, :1] + 1e-5 * base
+    mixed = base.copy()
+    mixed[:, 1::2] *= tiny**1.3
+    cases = [tiny * near, near / tiny, mixed, np.repeat(base[:, :1], n, axis=1), base]
+    t = _t(np.stack(cases), device, dtype)
+    h, tau, tblk = (x.cpu().double().numpy() for x in K.qr_factor(t))
+    nb = tblk.shape[-1]
+    for i in range(len(cases)):
+        q, wy = np.eye(m, n), np.eye(m, n)
+        v = np.tril(h[i], -1) + np.eye(m, n)
+        for j in reversed(range(n)):
+            q -= tau[i, j] * np.outer(v[:, j], v[:, j] @ q)
+        for p in reversed(range(tblk.shape[1])):
+            vp = v[:, p * nb: p * nb + nb]
+            wy -= vp @ (tblk[i, p][: vp.shape[1], : vp.shape[1]] @ (vp.T @ wy))
+        assert np.linalg.norm(wy - q, 2) <= m * n * u, i
+    # the columns left of equal ones shrink by u a step, and a double's squared
+    # norm (not a float's, which is a double) is below the smallest number then
+    for i in (3, 4) if dtype == torch.float32 else (4,):
+        _check_factor(t[i].cpu().double().numpy(), h[i], tau[i], tblk[i], u)
+
+
 @pytest.mark.parametrize("steps", [2, 3, 6])
 @pytest.mark.parametrize("shapes", [[(400, 90), (512, 130), (100, 200), (40, 33)],
                                     [(700, 300), (300, 200), (2100, 70), (33, 33)],
