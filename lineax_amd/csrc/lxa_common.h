@@ -5,6 +5,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <limits>
 
 #include "../../include/lineax_amd.h"
 
@@ -171,7 +172,9 @@ __device__ __forceinline__ bool plain_range(double d) { return fabs(d) >= 0x1p-9
 template <typename T>
 __device__ __forceinline__ T divide(T x, T d, T rd) {
   const T q = x * rd;
-  return fma(fma(-d, q, x), rd, q);
+  const T c = fma(fma(-d, q, x), rd, q);
+  // an infinite quotient has no correction (it would be inf - inf)
+  return fabs(q) <= std::numeric_limits<T>::max() ? c : q;
 }
 
 // Index of element (i, j), j >= i, in a row-packed upper triangle of order n.

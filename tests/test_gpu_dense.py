@@ -277,6 +277,21 @@ def test_cholesky_tiled_copies_agree(device, rng, n, dtype):
         assert torch.equal(u, alone.expand_as(u))
 
 
+@pytest.mark.parametrize("n", [65, 100, 181])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_solves_overflow_to_infinity(device, n, dtype):
+    """A quotient past the largest number is infinite, as a division gives it,
+    not NaN (the entries before the last one meet infinity times zero)."""
+    d = torch.eye(n, dtype=dtype, device=device)[None] * 1e-3
+    b = torch.zeros(1, n, dtype=dtype, device=device)
+    b[0, -1] = 0.9 * torch.finfo(dtype).max
+    piv = torch.arange(n, dtype=torch.int32, device=device)[None]
+    assert float(K.chol_solve(d, b)[0, -1]) == float("inf")
+    assert float(K.chol_solve(d, b, negate=True)[0, -1]) == -float("inf")
+    for trans in (0, 1):
+        assert float(K.lu_solve(d, piv, b, trans)[0, -1]) == float("inf")
+
+
 def test_gemv_matches(device, rng):
     # (5000, 300) and (4099, 37) split the transposed product over row chunks
     # (the 16-byte path and the scalar path); the rest run in one chunk
