@@ -551,7 +551,7 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
         const T zi = from_lane(z, i);
         if (ln > i) z -= m[i] * zi;
       }
-      if (lane < R) put(p * R + lane, z);
+      if (lane < R && p * R + lane < n) put(p * R + lane, z);  // padding stays 0, also beside infinities
     }
     barrier();
     if (c0 + (wv << 6) < n) {  // uniform
@@ -610,7 +610,7 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
         const T zi = from_lane(z, i);
         if (ln < i) z -= m[i] * zi;
       }
-      if (lane < R) put(p * R + lane, z);
+      if (lane < R && p * R + lane < n) put(p * R + lane, z);  // padding stays 0, also beside infinities
     }
     barrier();
     if (p > 0) {
