@@ -514,6 +514,18 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
   for (int h = 0; h < kSolveCols; ++h)
 #pragma unroll
     for (int i = 0; i < R; ++i) nx[h][i] = T(0);
+  // runs f(divide by this lane's diagonal entry of block p): by reciprocals, or
+  // as divisions where one of the block's entries has none that is normal
+  // (never a factor of lxa_chol_factor, whose entries are square roots)
+  auto chain = [&](int p, auto&& f) __attribute__((always_inline)) {
+    const T d = D[p & 1][lane % R][lane % R], r = rd[p & 1][lane % R];
+    const bool pad = p * R + lane % R >= n;
+    if (__all(pad || plain_range(d))) {
+      f([&](T z) { return z * r; });
+    } else {
+      f([&](T z) { return pad ? T(0) : z / d; });
+    }
+  };
   // the vector in global memory needs the barrier that orders global memory
   auto barrier = [&]() {
     if constexpr (InLds) {
@@ -541,16 +553,17 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
       T z = get(p * R + lane % R);
       int ln = lane % R;  // lanes past R repeat the others; opaque per block: lane masks are not held across blocks
       asm volatile("" : "+v"(ln));
-      const T r = rd[p & 1][lane % R];
       T m[R];
 #pragma unroll
       for (int i = 0; i < R; ++i) m[i] = D[p & 1][i][lane % R];
+      chain(p, [&](auto over) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < R; ++i) {
-        if (ln == i) z *= r;
-        const T zi = from_lane(z, i);
-        if (ln > i) z -= m[i] * zi;
-      }
+        for (int i = 0; i < R; ++i) {
+          if (ln == i) z = over(z);
+          const T zi = from_lane(z, i);
+          if (ln > i) z -= m[i] * zi;
+        }
+      });
       if (lane < R && p * R + lane < n) put(p * R + lane, z);  // padding stays 0, also beside infinities
     }
     barrier();
@@ -600,16 +613,17 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
         for (int w = 0; w < kSolveWaves; ++w) s += part[w][lane % R];
         z -= s;
       }
-      const T r = rd[p & 1][lane % R];
       T m[R];
 #pragma unroll
       for (int i = 0; i < R; ++i) m[i] = D[p & 1][lane % R][i];
+      chain(p, [&](auto over) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = R - 1; i >= 0; --i) {
-        if (ln == i) z *= r;
-        const T zi = from_lane(z, i);
-        if (ln < i) z -= m[i] * zi;
-      }
+        for (int i = R - 1; i >= 0; --i) {
+          if (ln == i) z = over(z);
+          const T zi = from_lane(z, i);
+          if (ln < i) z -= m[i] * zi;
+        }
+      });
       if (lane < R && p * R + lane < n) put(p * R + lane, z);  // padding stays 0, also beside infinities
     }
     barrier();

@@ -292,6 +292,23 @@ def test_solves_overflow_to_infinity(device, n, dtype):
         assert float(K.lu_solve(d, piv, b, trans)[0, -1]) == float("inf")
 
 
+@pytest.mark.parametrize("n", [100, 300])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_chol_solve_diagonals_without_reciprocal(device, rng, n, dtype):
+    """Factors given with subnormal or nearly largest diagonal entries: their
+    reciprocals are no normal numbers.  Each entry of the solution of a diagonal
+    factor is two divisions, rounded once each or to the smallest numbers' spacing."""
+    info = torch.finfo(dtype)
+    d, b = torch.ones(n, dtype=dtype), torch.from_numpy(rng.uniform(1, 2, n)).to(dtype)
+    for i in (3, n - 1):  # the solution there is a quarter of 1 / tiny
+        d[i], b[i] = info.tiny / 64, info.tiny / 2**14
+    d[n // 2], b[n // 2] = info.max / 2, info.max / 4
+    x = K.chol_solve(torch.diag(d).to(device)[None], b.to(device)[None])[0].cpu()
+    want = (b / d) / d
+    assert bool(torch.isfinite(want).all()) and float(want[3]) == 0.25 / info.tiny
+    assert bool(((x - want).abs() <= 2 * info.eps * want.abs() + info.tiny * info.eps).all())
+
+
 def test_gemv_matches(device, rng):
     # (5000, 300) and (4099, 37) split the transposed product over row chunks
     # (the 16-byte path and the scalar path); the rest run in one chunk
