@@ -120,9 +120,9 @@ class AbstractLinearSolver(abc.ABC):
 
 
 def _result_tensor(result, batch: tuple, device) -> torch.Tensor:
-    if not isinstance(result, torch.Tensor):
+    if isinstance(result, int):
         # filled on the device: a copy from the host would wait for the stream
-        return torch.full(batch, int(result), dtype=torch.int32, device=device)
+        return torch.full(batch, result, dtype=torch.int32, device=device)
     r = torch.as_tensor(result, dtype=torch.int32, device=device)
     return r.expand(batch).contiguous().clone() if r.shape != tuple(batch) else r.contiguous().clone()
 

@@ -74,6 +74,28 @@ def test_psd_tag_needs_square_structure():
         lx.MatrixLinearOperator(torch.ones(2, 3), lx.positive_semidefinite_tag)
 
 
+@pytest.mark.parametrize("codes", [0, [0, 2], (0, 2), np.array([0, 2]), np.int64(2), torch.tensor([0, 2])])
+def test_solver_result_codes_in_any_form(codes):
+    """A solver may return its codes as one number, a list, an array or a tensor."""
+
+    class Given(lx.AbstractLinearSolver):
+        def init(self, operator, options):
+            return None
+
+        def compute(self, state, vector, options):
+            return vector, codes, {}
+
+        transpose = conj = assume_full_rank = None
+
+    op = lx.MatrixLinearOperator(torch.eye(3).expand(2, 3, 3))
+    want = torch.as_tensor(codes).expand(2).tolist()
+    sol = lx.linear_solve(op, torch.ones(2, 3), Given(), throw=False)
+    assert sol.result.dtype == torch.int32 and sol.result.tolist() == want
+    if any(want):
+        with pytest.raises(RuntimeError, match="non-finite"):
+            lx.linear_solve(op, torch.ones(2, 3), Given())
+
+
 def test_linear_solve_validation():
     with pytest.raises(ValueError, match="raw tensor"):
         lx.linear_solve(torch.eye(2), torch.ones(2))
