@@ -311,14 +311,14 @@ __global__ __launch_bounds__(kBigThreads) void qr_apply_kernel(const lxa_qr_desc
 // The same product for systems of up to kApplyMaxRows rows, one vector per
 // workgroup: the vector lives in LDS and NB lanes share a row (lane j reads
 // column j of the panel, so a wave load covers 64 / NB contiguous row
-// segments instead of 64 scattered ones).  RPT > 0: each lane keeps its
-// RPT panel entries in registers between the reduction and the update (V is
-// read once per panel); RPT == 0 reads them twice.  Per panel:
+// segments instead of 64 scattered ones).  Each lane keeps its entries of the
+// first RPT passes' rows in registers between the reduction and the update;
+// REST: there may be further rows, which are read twice.  Per panel:
 //   w = V^T x (lanes of a column, then waves, summed in a fixed order);
-//   w = T^T w or T w (wave 0, shuffles);  x -= V w (row sums of up to 16 rows
+//   w = T^T w or T w (wave 0, shuffles);  x -= V w (row sums of 8 or 16 rows
 //   at a time by a reduce-scatter over their 16 lanes).
-// One double system of 3001 x 391, its panels read twice in rounds of eight
-// rows and a four-step butterfly per row: 763 us.
+// One compute unit reading V bounds it.  A double system of 3001 x 391: 429 us;
+// all rows read twice with a four-step butterfly per row 764 us.
 // ---------------------------------------------------------------------------
 constexpr int kApplyMaxRows = 16384;
 
@@ -344,18 +344,17 @@ __device__ __forceinline__ T row_reduce_scatter(T (&v)[K], int j) {
   }
 }
 
-template <typename T, int RPT, int WAVES>
-__global__ __launch_bounds__(WAVES * kWave) void qr_apply_rows_kernel(const lxa_qr_desc* __restrict__ descs,
-                                                                      const T* __restrict__ a,
-                                                                      const T* __restrict__ tblk,
-                                                                      T* __restrict__ b, int trans) {
+template <typename T, int RPT, bool REST>
+__global__ __launch_bounds__(kBigThreads) void qr_apply_rows_kernel(const lxa_qr_desc* __restrict__ descs,
+                                                                    const T* __restrict__ a,
+                                                                    const T* __restrict__ tblk,
+                                                                    T* __restrict__ b, int trans) {
   constexpr int NB = QrCfg<T>::NB;
   constexpr int G = kWave / NB;       // rows per wave load
-  constexpr int RP = WAVES * G;       // rows per pass of the workgroup
-  constexpr int kBlock = WAVES * kWave;
+  constexpr int RP = kBigWaves * G;   // rows per pass of the workgroup
   extern __shared__ __align__(16) unsigned char apply_smem[];
   T* xs = reinterpret_cast<T*>(apply_smem);
-  __shared__ T s_part[WAVES][NB];
+  __shared__ T s_part[kBigWaves][NB];
   __shared__ T s_w[NB];
   const lxa_qr_desc d = descs[blockIdx.x];
   const int m = d.m, lda = d.lda;
@@ -365,7 +364,7 @@ __global__ __launch_bounds__(WAVES * kWave) void qr_apply_rows_kernel(const lxa_
   const int j = lane % NB, rg = wv * G + lane / NB;
   const T* A = a + d.a_offset;
   T* x = b + d.b_offset + (int64_t)blockIdx.y * d.ldb;
-  for (int i = tid; i < m; i += kBlock) xs[i] = x[i];
+  for (int i = tid; i < m; i += kBigThreads) xs[i] = x[i];
   __syncthreads();
   const int panels = (kmax + NB - 1) / NB;
   T v[RPT > 0 ? RPT : 1];
@@ -398,9 +397,10 @@ __global__ __launch_bounds__(WAVES * kWave) void qr_apply_rows_kernel(const lxa_
         const int row = k + rg + t * RP;
         if (row < m) acc += v[t] * xs[row];
       }
-    } else {
+    }
+    if constexpr (REST) {
       // eight rows per round, loads issued together (clamped rows, masked)
-      for (int row0 = k + rg; row0 < m; row0 += 8 * RP) {
+      for (int row0 = k + rg + RPT * RP; row0 < m; row0 += 8 * RP) {
         T st[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) st[u] = Ak[(int64_t)min(row0 + u * RP, m - 1) * lda];
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(WAVES * kWave) void qr_apply_rows_kernel(const lxa_
       T wsum = T(0);
       if (lane < NB) {
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) wsum += s_part[w][lane];
+        for (int w = 0; w < kBigWaves; ++w) wsum += s_part[w][lane];
       }
       T s = T(0);
 #pragma unroll
@@ -448,34 +448,35 @@ __global__ __launch_bounds__(WAVES * kWave) void qr_apply_rows_kernel(const lxa_
         const int row = k + rg + (t0 + j / (NB / K)) * RP;
         if (j % (NB / K) == 0 && row < m) xs[row] -= sum;
       }
-    } else {
-      for (int row0 = k + rg; row0 < m; row0 += 8 * RP) {
+    }
+    if constexpr (REST) {
+      for (int row0 = k + rg + RPT * RP; row0 < m; row0 += 8 * RP) {
         T st[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) st[u] = Ak[(int64_t)min(row0 + u * RP, m - 1) * lda];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
           const int row = row0 + u * RP;
-          T s = (row < m && j < nb) ? vpick(row, k + j, st[u]) * wj : T(0);
-#pragma unroll
-          for (int off = 1; off < NB; off <<= 1) s += __shfl_xor(s, off, kWave);
-          if (j == 0 && row < m) xs[row] -= s;
+          st[u] = (row < m && j < nb) ? vpick(row, k + j, st[u]) * wj : T(0);
         }
+        const T sum = row_reduce_scatter<8>(st, j);
+        const int row = row0 + j / 2 * RP;
+        if (j % 2 == 0 && row < m) xs[row] -= sum;
       }
     }
     __syncthreads();
   }
-  for (int i = tid; i < m; i += kBlock) x[i] = xs[i];
+  for (int i = tid; i < m; i += kBigThreads) x[i] = xs[i];
 }
 
-template <typename T, int RPT, int WAVES>
+template <typename T, int RPT, bool REST>
 int launch_apply_rows(hipStream_t st, dim3 grid, int max_m, const lxa_qr_desc* desc, const void* a, const void* tblk,
                       void* b, int trans) {
   const size_t smem = sizeof(T) * (size_t)max_m;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&qr_apply_rows_kernel<T, RPT, WAVES>),
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&qr_apply_rows_kernel<T, RPT, REST>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (e != hipSuccess) return hip_error(e, "hipFuncSetAttribute(qr_apply_rows)");
-  qr_apply_rows_kernel<T, RPT, WAVES><<<grid, WAVES * kWave, smem, st>>>(
+  qr_apply_rows_kernel<T, RPT, REST><<<grid, kBigThreads, smem, st>>>(
       desc, static_cast<const T*>(a), static_cast<const T*>(tblk), static_cast<T*>(b), trans);
   LXA_LAUNCH_CHECK("qr_apply_rows_kernel");
   return LXA_OK;
@@ -484,16 +485,18 @@ int launch_apply_rows(hipStream_t st, dim3 grid, int max_m, const lxa_qr_desc* d
 template <typename T>
 int apply_rows(hipStream_t st, dim3 grid, int max_m, const lxa_qr_desc* desc, const void* a, const void* tblk,
                void* b, int trans) {
-  // 16 waves up to 16 panel entries per lane (128 registers each), then eight
-  // waves, which have 256: up to 2048 rows, then as many as they hold
-  constexpr int kPass = kWave / QrCfg<T>::NB;  // rows per wave load
-  constexpr int kMost = sizeof(T) == 4 ? 128 : 96;
-  if (max_m <= 4 * 16 * kPass) return launch_apply_rows<T, 4, 16>(st, grid, max_m, desc, a, tblk, b, trans);
-  if (max_m <= 8 * 16 * kPass) return launch_apply_rows<T, 8, 16>(st, grid, max_m, desc, a, tblk, b, trans);
-  if (max_m <= 16 * 16 * kPass) return launch_apply_rows<T, 16, 16>(st, grid, max_m, desc, a, tblk, b, trans);
-  if (max_m <= 64 * 8 * kPass) return launch_apply_rows<T, 64, 8>(st, grid, max_m, desc, a, tblk, b, trans);
-  if (max_m <= kMost * 8 * kPass) return launch_apply_rows<T, kMost, 8>(st, grid, max_m, desc, a, tblk, b, trans);
-  return launch_apply_rows<T, 0, 16>(st, grid, max_m, desc, a, tblk, b, trans);
+  // 16 waves of 128 registers hold 16 panel entries a lane, 1024 rows; a system
+  // of 1500 x 391 takes 131 us (float) / 223 us (double) so, 167 / 290 us with
+  // 64 entries in eight waves, of 3001 rows 288 / 429 us and, with the 128 / 96
+  // entries that eight waves cannot hold, 574 / 674 us.  Above 4096 rows the
+  // 1024 are too few to matter: 8000 x 100 185 / 290 us with them, 171 / 288 us
+  // without.
+  constexpr int kPass = 16 * (kWave / QrCfg<T>::NB);  // rows per pass of 16 waves
+  if (max_m <= 4 * kPass) return launch_apply_rows<T, 4, false>(st, grid, max_m, desc, a, tblk, b, trans);
+  if (max_m <= 8 * kPass) return launch_apply_rows<T, 8, false>(st, grid, max_m, desc, a, tblk, b, trans);
+  if (max_m <= 16 * kPass) return launch_apply_rows<T, 16, false>(st, grid, max_m, desc, a, tblk, b, trans);
+  if (max_m <= 4096) return launch_apply_rows<T, 16, true>(st, grid, max_m, desc, a, tblk, b, trans);
+  return launch_apply_rows<T, 0, true>(st, grid, max_m, desc, a, tblk, b, trans);
 }
 
 // ---------------------------------------------------------------------------

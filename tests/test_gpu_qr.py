@@ -256,6 +256,35 @@ def test_qr_transpose_state_reuse(device, rng):
     np.testing.assert_allclose(x_t.cpu().numpy(), np.linalg.lstsq(a.T, c, rcond=None)[0], rtol=1e-10, atol=1e-10)
 
 
+@pytest.mark.parametrize("m,n", [(1, 1), (255, 40), (257, 33), (512, 20), (513, 48), (1024, 30), (1025, 17), (1041, 100),
+                                 (2049, 16), (3001, 70), (4096, 15), (4097, 33), (9000, 20), (16385, 18)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_qr_apply_edges(device, rng, m, n, dtype):
+    """Heights around the rows that are kept in registers, those read twice and
+    the form without LDS; both directions, two right-hand sides.  The error
+    against 64 bits is at most four times that of the reflectors applied one
+    after the other in the same precision, plus four roundings."""
+    nb, u = K.qr_block(dtype), torch.finfo(dtype).eps / 2
+    a, tau, tblk = K.qr_factor(_t(rng.standard_normal((m, n)), device, dtype))
+    b = _t(rng.standard_normal((2, m)), device, dtype)
+    d = np.zeros(1, dtype=K.QR_DESC)
+    d["m"], d["n"], d["lda"], d["ldb"] = m, n, n, m
+    h, t = a.cpu().numpy(), tau.cpu().numpy()
+    v = np.tril(h, -1)
+    v[np.arange(n), np.arange(n)] = 1
+    for trans in (True, False):
+        got = b.clone()
+        K.qr_apply_raw(K.descs_to_device(d, device), 1, m, n, a, tblk, 2, got, trans=trans)
+        same, wide = b.cpu().numpy().T.copy(), b.cpu().double().numpy().T.copy()
+        for j in range(n) if trans else reversed(range(n)):
+            same -= t[j] * np.outer(v[:, j], v[:, j] @ same)
+            vj = v[:, j].astype(np.float64)
+            wide -= float(t[j]) * np.outer(vj, vj @ wide)
+        scale = np.linalg.norm(wide)
+        limit = 4 * np.linalg.norm(same - wide) / scale + 4 * u
+        assert np.linalg.norm(got.cpu().double().numpy().T - wide) / scale <= limit
+
+
 def test_qr_solve_refuses_other_t_blocks(device, rng):
     """T blocks that are not the factor's (8-wide ones, of another order or
     batch) are an error on the host, not reads past their end."""
