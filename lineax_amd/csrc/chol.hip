@@ -370,12 +370,16 @@ int chol_factor_t(hipStream_t s, int64_t batch, int64_t n64, T* a, int64_t strid
   else if (n <= 16) launch_chol_small<T, 16>(s, batch, n, a, stride, negate, info);
   else if (n <= 32) launch_chol_small<T, 32>(s, batch, n, a, stride, negate, info);
   else if (n <= 64) launch_chol_small<T, 64>(s, batch, n, a, stride, negate, info);
-  else if (sizeof(T) == 8 && n <= kLdsFactorMax && batch > kLdsFactorBatch) {
-    const size_t shmem = static_cast<size_t>(n) * (n + 1) / 2 * sizeof(T);
-    if (int rc = allow_lds(chol_factor_lds_kernel<T>, shmem)) return rc;
-    hipLaunchKernelGGL((chol_factor_lds_kernel<T>), dim3(static_cast<unsigned>(batch)), dim3(kWG), shmem, s, n, a,
-                       stride, negate, info);
-  } else {
+  else {
+    if constexpr (sizeof(T) == 8) {
+      if (n <= kLdsFactorMax && batch > kLdsFactorBatch) {
+        const size_t shmem = static_cast<size_t>(n) * (n + 1) / 2 * sizeof(T);
+        hipLaunchKernelGGL((chol_factor_lds_kernel<T>), dim3(static_cast<unsigned>(batch)), dim3(kWG), shmem, s, n, a,
+                           stride, negate, info);
+        LXA_LAUNCH_CHECK("lxa_chol_factor launch");
+        return LXA_OK;
+      }
+    }
     return chol_tile_factor(s, batch, n, a, stride, negate, info);
   }
   LXA_LAUNCH_CHECK("lxa_chol_factor launch");

@@ -219,13 +219,15 @@ def test_cholesky_reads_upper_triangle_only(device, rng, n, dtype):
 
 
 @pytest.mark.parametrize("n,dtype", [
+    (65, torch.float32), (128, torch.float32), (129, torch.float32), (193, torch.float32), (256, torch.float32),
+    (65, torch.float64), (127, torch.float64), (128, torch.float64), (129, torch.float64), (181, torch.float64),
     (257, torch.float32), (319, torch.float32), (320, torch.float32), (321, torch.float32), (577, torch.float32),
     (182, torch.float64), (192, torch.float64), (193, torch.float64), (256, torch.float64), (449, torch.float64),
     (1100, torch.float64),
 ])
 def test_cholesky_tiled(device, rng, n, dtype):
-    """Orders around the 64-row tiles, past 1024 columns (two per thread in the
-    solve), either sign, garbage below the diagonal, a batch of which one fails.
+    """Orders around the 64-row tiles and the LDS solve's limits (256 in float, 181
+    in double), past 1024 columns (two per thread in the tiled solve), either sign, garbage below the diagonal, a batch of which one fails.
 
     Bounds: |U^T U - A| <= gamma_(n+1) |U|^T |U| componentwise (Higham, Accuracy
     and Stability, thm 10.3; the row norms of |U|^T |U| are below max a_ii), and
@@ -260,6 +262,61 @@ def test_cholesky_tiled(device, rng, n, dtype):
         r = (exact @ x[:2, :, None])[..., 0] - rhs[:2].cpu().double()
         scale = (uc.abs().mT @ (uc.abs() @ x[:2, :, None].abs()))[..., 0]
         assert bool((r.abs() <= 2 * (3 * n + 2) * eps * scale).all())
+
+
+@pytest.mark.parametrize("n,batch", [(64, 513), (65, 513), (80, 513), (96, 513), (96, 512), (97, 513)])
+@pytest.mark.parametrize("negate", [False, True])
+def test_cholesky_many_small_doubles(device, rng, n, batch, negate):
+    """Orders 65..96 in batches above 512 have a kernel of their own; either side
+    of its limits, garbage below the diagonal, failing systems first, last and in
+    between.  Bounds as in test_cholesky_tiled."""
+    eps = torch.finfo(torch.float64).eps / 2
+    base = np.stack([well_conditioned(rng, n, kind="psd") for _ in range(8)])
+    mats = base[np.arange(batch) % 8]
+    fails = {0: n // 2, 257: n - 1, batch - 1: 0}
+    for s, at in fails.items():
+        mats[s, at, at] = -1.0
+    given = np.where(np.tri(n, k=-1, dtype=bool), 1e30, -mats if negate else mats)
+    u, info = K.chol_factor(_t(given, device), negate=negate)
+    assert {i: int(x) - 1 for i, x in enumerate(info.tolist()) if x} == fails
+    x = K.chol_solve(u, _t(np.ones((batch, n)), device), negate=negate).cpu()
+    u = u.cpu()
+    for s in range(batch):
+        if s in fails:
+            assert bool(torch.isnan(u[s]).all()) and bool(torch.isnan(x[s]).all())
+            continue
+        assert bool((torch.tril(u[s], -1) == 0).all())
+        exact = torch.from_numpy(mats[s])
+        grown = u[s].abs().mT @ u[s].abs()
+        assert bool(((u[s].mT @ u[s] - exact).abs() <= 2 * (n + 2) * eps * grown).all())
+        r = exact @ (-x[s] if negate else x[s]) - 1.0
+        assert bool((r.abs() <= 2 * (3 * n + 2) * eps * (grown @ x[s].abs())).all())
+
+
+@pytest.mark.parametrize("n,dtype", [(16400, torch.float64), (20480, torch.float64), (32800, torch.float32)])
+def test_chol_solve_vector_in_global_memory(device, rng, n, dtype):
+    """Orders whose vector does not fit in LDS, with a banded factor: the bound on
+    the backward error of the solve (Higham, Accuracy and Stability, thm 8.5 for
+    each triangle) has the band's five entries a row and column."""
+    eps = torch.finfo(dtype).eps / 2
+    band = {0: 2.0 + rng.random(n), 1: rng.standard_normal(n - 1) / 2, 37: rng.standard_normal(n - 37) / 2,
+            n // 2: rng.standard_normal(n - n // 2) / 2, n - 3: rng.standard_normal(3) / 2}
+    u = torch.zeros(n, n, dtype=dtype, device=device)
+    for k, v in band.items():
+        torch.diagonal(u, k).copy_(_t(v, device, dtype))
+    b = _t(rng.standard_normal(n), device, dtype)
+    x = K.chol_solve(u[None], b[None])[0].double().cpu().numpy()
+    band = {k: torch.diagonal(u, k).double().cpu().numpy() for k in band}
+
+    def upper(d, v):  # U v
+        return sum(np.concatenate([d[k] * v[k:], np.zeros(k)]) for k in d)
+
+    def lower(d, v):  # U^T v
+        return sum(np.concatenate([np.zeros(k), d[k] * v[: n - k]]) for k in d)
+
+    size = {k: np.abs(v) for k, v in band.items()}
+    r = np.abs(lower(band, upper(band, x)) - b.double().cpu().numpy())
+    assert np.all(r <= 2 * 3 * (len(band) + 2) * eps * lower(size, upper(size, np.abs(x))))
 
 
 @pytest.mark.parametrize("n,dtype", [(80, torch.float32), (200, torch.float32), (256, torch.float32),
