@@ -122,7 +122,8 @@ class Arena:
 def qr_footprint(m: int, n: int, nb: int = 16) -> dict:
     """Arena elements of one QR system: matrix, tau, T blocks, scratch, rhs."""
     k = min(m, n)
-    return {"a": m * n, "tau": k, "t": -(-k // nb) * nb * nb, "w": -(-m // 256) * nb * n, "b": m}
+    return {"a": m * n, "tau": k, "t": -(-k // nb) * nb * nb,
+            "w": K.qr_work_elems(torch.float32, m, n), "b": m}
 
 
 def chol_footprint(n: int) -> dict:

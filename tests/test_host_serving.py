@@ -1,7 +1,10 @@
 """Host logic of the request loop: the HBM arena and the request stream."""
 
 import numpy as np
+import pytest
+import torch
 
+from lineax_amd import _kernels as K
 from lineax_amd import serving as S
 
 
@@ -31,6 +34,14 @@ def test_arena_first_fit_and_coalescing():
     for off, n in list(live.values()):
         ar.release(off, n)
     assert ar.free == [(0, ar.size)] and ar.used == 0
+
+
+def test_qr_footprint_is_what_the_kernels_use():
+    if not K.LIB_PATH.exists():
+        pytest.skip("kernel library not built")
+    fp = S.qr_footprint(4096, 1001)
+    assert fp == {"a": 4096 * 1001, "tau": 1001, "t": 63 * 256, "w": K.qr_work_elems(torch.float32, 4096, 1001),
+                  "b": 4096}
 
 
 def test_request_stream_statistics():
