@@ -145,16 +145,6 @@ __global__ __launch_bounds__(64) void chol_solve_small_kernel(int64_t batch, int
 // ---------------------------------------------------------------------------
 constexpr int kWG = 256;
 
-__device__ __forceinline__ float bcast_lane(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-__device__ __forceinline__ double bcast_lane(double v, int lane) {
-  const int64_t bits = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane(static_cast<int>(bits & 0xffffffff), lane);
-  const int hi = __builtin_amdgcn_readlane(static_cast<int>(bits >> 32), lane);
-  return __longlong_as_double((static_cast<int64_t>(hi) << 32) | static_cast<uint32_t>(lo));
-}
-
 // Loads the upper triangle of A (row-major, leading dimension lda) into the
 // row-packed LDS triangle L.  Wave w takes rows w, w+4, ...; lanes cover the
 // columns, and four rows are in flight per wave.
@@ -254,7 +244,7 @@ __device__ void wave_chol_solve(int n, const T* L, T (&v)[4]) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) cur[c] = nxt[c];
       row(k + 1, nxt);
-      const T yk = bcast_lane(over(v[c0], c0), kk);
+      const T yk = from_lane(over(v[c0], c0), kk);
       if (l == kk) v[c0] = yk;
 #pragma unroll
       for (int c = c0; c < 4; ++c)
@@ -276,7 +266,7 @@ __device__ void wave_chol_solve(int n, const T* L, T (&v)[4]) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) cur[c] = nxt[c];
       column(k - 1, nxt);
-      const T xk = bcast_lane(over(v[c0], c0), kk);
+      const T xk = from_lane(over(v[c0], c0), kk);
       if (l == kk) v[c0] = xk;
 #pragma unroll
       for (int c = 0; c <= c0; ++c)

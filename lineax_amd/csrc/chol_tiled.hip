@@ -38,46 +38,6 @@ constexpr int kS = 16;        // strip
 constexpr int kThreads = 256;
 constexpr int kLd = 2 * kT + 2;  // LDS row: diagonal tile, then the solved tile
 
-template <typename T>
-struct Mma;
-// One 16 x 16 x 4 matrix-core product.  Lane l: A operand [l % 16][l / 16],
-// B operand [l / 16][l % 16]; row(l, i) is the result row of register i, the
-// column is l % 16.
-template <>
-struct Mma<float> {
-  typedef float acc __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ acc mul(float a, float b, acc c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int l, int i) { return 4 * (l >> 4) + i; }
-};
-template <>
-struct Mma<double> {
-  typedef double acc __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ acc mul(double a, double b, acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int l, int i) { return (l >> 4) + 4 * i; }
-};
-
-__device__ __forceinline__ float from_lane(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-__device__ __forceinline__ double from_lane(double v, int lane) {
-  const int64_t bits = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane(static_cast<int>(bits & 0xffffffff), lane);
-  const int hi = __builtin_amdgcn_readlane(static_cast<int>(bits >> 32), lane);
-  return __longlong_as_double((static_cast<int64_t>(hi) << 32) | static_cast<uint32_t>(lo));
-}
-
-template <int B, int E, typename F>
-__device__ __forceinline__ void unroll(F&& f) {
-  if constexpr (B < E) {
-    f(std::integral_constant<int, B>{});
-    unroll<B + 1, E>(f);
-  }
-}
-
 // Square root and its reciprocal of a pivot, from the hardware reciprocal
 // square root and Newton steps (the correctly rounded sqrt and division cost
 // about four times as many dependent instructions on the chain): within an
@@ -192,7 +152,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 2) void chol_tile_ke
     fetch_rows(A, ld, n, k0 - kT, j * kT, vj);
     M4 acc[4];
     {
-      int row = min(i * kT + 16 * wv + Mma<T>::row(lane, 0), n - 1);
+      int row = min(i * kT + 16 * wv + Mma<T>::row(g, 0), n - 1);
       const T* p = A + (int64_t)row * ld;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -215,7 +175,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 2) void chol_tile_ke
     }
     {
       const bool whole = i < j && j + 1 < nt;  // uniform
-      int row = i * kT + 16 * wv + Mma<T>::row(lane, 0);
+      int row = i * kT + 16 * wv + Mma<T>::row(g, 0);
       T* p = A + (int64_t)row * ld;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -246,7 +206,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 2) void chol_tile_ke
       if (kTiles == 8) fetch_rows(A, ld, n, k0 - kT, j * kT, vj);
     }
     M4 acc[kTiles];
-    int row = min(k0 + 16 * wv + Mma<T>::row(lane, 0), n - 1);
+    int row = min(k0 + 16 * wv + Mma<T>::row(g, 0), n - 1);
     const T* p = A + (int64_t)row * ld;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -257,7 +217,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 2) void chol_tile_ke
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int r = 16 * wv + Mma<T>::row(lane, e);
+      const int r = 16 * wv + Mma<T>::row(g, e);
 #pragma unroll
       for (int c = 0; c < kTiles; ++c) {
         const int cl = 16 * (c & 3) + q;
@@ -284,7 +244,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 2) void chol_tile_ke
 #pragma unroll
     for (int c = 0; c < kTiles; ++c) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) M[(16 * wv + Mma<T>::row(lane, e)) * kLd + 16 * c + q] = acc[c][e];
+      for (int e = 0; e < 4; ++e) M[(16 * wv + Mma<T>::row(g, e)) * kLd + 16 * c + q] = acc[c][e];
     }
   };
   if (j > k) {
@@ -313,7 +273,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 2) void chol_tile_ke
       asm volatile("" : "+v"(ln));
 #pragma unroll
       for (int i = 0; i < kS; ++i) c[i] = Ms[i * kLd];
-      unroll<0, kS>([&](auto T_) __attribute__((always_inline)) {
+      static_for<0, kS>([&](auto T_) __attribute__((always_inline)) {
         constexpr int p = decltype(T_)::value;
         const T d = from_lane(c[p], p);
         if (!(d > T(0)) && fail == 0) fail = k0 + r0 + p + 1;
@@ -325,7 +285,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 2) void chol_tile_ke
           inv = T(1) / u;
         }
         c[p] = ln == p ? u : c[p] * inv;
-        unroll<p + 1, kS>([&](auto I_) __attribute__((always_inline)) {
+        static_for<p + 1, kS>([&](auto I_) __attribute__((always_inline)) {
           constexpr int i = decltype(I_)::value;
           c[i] -= from_lane(c[p], i) * c[p];
         });
@@ -354,14 +314,14 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 2) void chol_tile_ke
         M4 acc;
         T* Mt = M + 16 * r * kLd + 16 * c + q;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] = Mt[Mma<T>::row(lane, e) * kLd];
+        for (int e = 0; e < 4; ++e) acc[e] = Mt[Mma<T>::row(g, e) * kLd];
 #pragma unroll
         for (int h = 0; h < kS; h += 4) {
           const T* Mh = M + (r0 + h + g) * kLd;
           acc = Mma<T>::mul(-Mh[16 * r + q], Mh[16 * c + q], acc);
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) Mt[Mma<T>::row(lane, e) * kLd] = acc[e];
+        for (int e = 0; e < 4; ++e) Mt[Mma<T>::row(g, e) * kLd] = acc[e];
       }
       idx -= cnt;
     }

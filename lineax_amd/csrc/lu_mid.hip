@@ -33,46 +33,6 @@ constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / kWave;
 constexpr int kLpLd = kP + 1;  // row stride of the staged L21
 
-template <typename T>
-struct Mma;
-// One 16 x 16 x 4 matrix-core product.  Lane l: A operand [l % 16][l / 16],
-// B operand [l / 16][l % 16]; row(l, i) is the result row of register i, the
-// column is l % 16.
-template <>
-struct Mma<float> {
-  typedef float acc __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ acc mul(float a, float b, acc c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int l, int i) { return 4 * (l >> 4) + i; }
-};
-template <>
-struct Mma<double> {
-  typedef double acc __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ acc mul(double a, double b, acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int l, int i) { return (l >> 4) + 4 * i; }
-};
-
-__device__ __forceinline__ float from_lane(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-__device__ __forceinline__ double from_lane(double v, int lane) {
-  const int64_t bits = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane(static_cast<int>(bits & 0xffffffff), lane);
-  const int hi = __builtin_amdgcn_readlane(static_cast<int>(bits >> 32), lane);
-  return __longlong_as_double((static_cast<int64_t>(hi) << 32) | static_cast<uint32_t>(lo));
-}
-
-template <int B, int E, typename F>
-__device__ __forceinline__ void unroll(F&& f) {
-  if constexpr (B < E) {
-    f(std::integral_constant<int, B>{});
-    unroll<B + 1, E>(f);
-  }
-}
-
 // Order of |v| with NaN largest, in 32-bit words: high, then low.
 __device__ __forceinline__ unsigned key_hi(float v) { return __float_as_uint(v) & 0x7fffffffu; }
 __device__ __forceinline__ unsigned key_hi(double v) {
@@ -136,7 +96,7 @@ __global__ __launch_bounds__(kThreads) void lu_mid_factor_kernel(int n, T* __res
         for (int c = 0; c < kP; ++c)
           if (done[s] || c >= w) row[s][c] = T(0);
       }
-      unroll<0, kP>([&](auto T_) __attribute__((always_inline)) {
+      static_for<0, kP>([&](auto T_) __attribute__((always_inline)) {
         constexpr int t = decltype(T_)::value;
         if (t >= w) return;  // uniform
         // largest |a_ik| over the remaining rows, ties to the smallest position
@@ -238,7 +198,7 @@ __global__ __launch_bounds__(kThreads) void lu_mid_factor_kernel(int n, T* __res
         d[t] = W[(k0 + tt) * ld + c];
       }
       if (c >= k0 + w) {
-        unroll<0, kP>([&](auto T_) __attribute__((always_inline)) {
+        static_for<0, kP>([&](auto T_) __attribute__((always_inline)) {
           constexpr int t = decltype(T_)::value;
 #pragma unroll
           for (int i = t + 1; i < kP; ++i) v[i] -= s_l11[i][t] * v[t];
@@ -271,7 +231,7 @@ __global__ __launch_bounds__(kThreads) void lu_mid_factor_kernel(int n, T* __res
         for (int u = 0; u < 4; ++u) {
           const int col = min(base + 16 * (ct + u) + q, n - 1);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[u][e] = W[min(r0 + Mma<T>::row(lane, e), n - 1) * ld + col];
+          for (int e = 0; e < 4; ++e) acc[u][e] = W[min(r0 + Mma<T>::row(g, e), n - 1) * ld + col];
         }
         const int lr = min(r0 + q, n - 1);
 #pragma unroll
@@ -289,7 +249,7 @@ __global__ __launch_bounds__(kThreads) void lu_mid_factor_kernel(int n, T* __res
           const int col = base + 16 * (ct + u) + q;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const int r = r0 + Mma<T>::row(lane, e);
+            const int r = r0 + Mma<T>::row(g, e);
             if (r < n && col < n) W[r * ld + col] = acc[u][e];
           }
         }

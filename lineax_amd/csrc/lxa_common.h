@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstdint>
 #include <limits>
+#include <type_traits>
 
 #include "../../include/lineax_amd.h"
 
@@ -123,6 +124,50 @@ __device__ __forceinline__ T lane_xor(T v) {
     return __builtin_bit_cast(T, (static_cast<unsigned long long>(hi) << 32) | lo);
   }
 }
+
+// f(std::integral_constant<int, B>) .. f(<E - 1>): a loop whose index is a
+// compile-time constant (register arrays indexed by it stay in registers).
+template <int B, int E, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    static_for<B + 1, E>(f);
+  }
+}
+
+// The value of one lane of the wave (uniform index) in every lane, through
+// scalar registers.
+__device__ __forceinline__ float from_lane(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ double from_lane(double v, int lane) {
+  const int64_t bits = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane(static_cast<int>(bits & 0xffffffff), lane);
+  const int hi = __builtin_amdgcn_readlane(static_cast<int>(bits >> 32), lane);
+  return __longlong_as_double((static_cast<int64_t>(hi) << 32) | static_cast<uint32_t>(lo));
+}
+
+// One 16 x 16 x 4 matrix-core product.  Lane l = 16 g + q: A operand
+// [q][inner g], B operand [inner g][q]; result register e holds row row(g, e)
+// and column q.
+template <typename T>
+struct Mma;
+template <>
+struct Mma<float> {
+  typedef float acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mul(float a, float b, acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ constexpr int row(int g, int e) { return 4 * g + e; }
+};
+template <>
+struct Mma<double> {
+  typedef double acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mul(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ constexpr int row(int g, int e) { return g + 4 * e; }
+};
 
 // One halving level of wave_reduce_scatter, and the levels after it: lanes
 // with bit `off` set keep the upper half of v and add their partner's upper

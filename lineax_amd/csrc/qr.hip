@@ -529,17 +529,6 @@ int apply_rows(hipStream_t st, dim3 grid, int max_m, const lxa_qr_desc* desc, co
 constexpr int kTrsvBlock = 64;
 constexpr int kTrsvMaxK = 8192;
 
-// v from lane j of the wave (j uniform): v_readlane into a scalar register.
-__device__ __forceinline__ float lane_bcast(float v, int j) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
-}
-__device__ __forceinline__ double lane_bcast(double v, int j) {
-  const long long bits = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane(static_cast<int>(bits), j);
-  const int hi = __builtin_amdgcn_readlane(static_cast<int>(bits >> 32), j);
-  return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-}
-
 template <typename T>
 __global__ __launch_bounds__(kBigThreads) void trsv_kernel(const lxa_qr_desc* __restrict__ descs,
                                                              const T* __restrict__ a, T* __restrict__ b, int lower,
@@ -638,7 +627,7 @@ __global__ __launch_bounds__(kBigThreads) void trsv_kernel(const lxa_qr_desc* __
         for (int j = kTrsvBlock - 1; j >= 0; --j) {
           const T mult = tile[lane * (kTrsvBlock + 1) + j];
           if (lane == j) z *= rl;
-          const T xj = j < bs ? lane_bcast(z, j) : T(0);
+          const T xj = j < bs ? from_lane(z, j) : T(0);
           if (lane < j) z -= mult * xj;
         }
       } else {
@@ -646,7 +635,7 @@ __global__ __launch_bounds__(kBigThreads) void trsv_kernel(const lxa_qr_desc* __
         for (int j = 0; j < kTrsvBlock; ++j) {
           const T mult = tile[j * (kTrsvBlock + 1) + lane];
           if (lane == j) z *= rl;
-          const T xj = j < bs ? lane_bcast(z, j) : T(0);
+          const T xj = j < bs ? from_lane(z, j) : T(0);
           if (lane > j) z -= mult * xj;
         }
       }

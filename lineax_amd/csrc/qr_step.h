@@ -1,8 +1,6 @@
 // What the QR panel step kernels (qr_step_*.hip) and the
 // factorisation around them (qr.hip) share.
 #pragma once
-#include <type_traits>
-
 #include "lxa_common.h"
 
 namespace lxa {
@@ -36,14 +34,6 @@ struct QrCfg {
 
 constexpr int kPanelThreads = 512;   // 2 waves per SIMD: 256 VGPRs each
 constexpr int kPanelWaves = kPanelThreads / kWave;
-
-template <int B, int E, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (B < E) {
-    f(std::integral_constant<int, B>{});
-    static_for<B + 1, E>(f);
-  }
-}
 
 // Householder vector entry j of panel-relative row (row - k): 1 on the
 // diagonal, the stored value below it, 0 above.

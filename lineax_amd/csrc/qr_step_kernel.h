@@ -13,29 +13,9 @@ namespace {
 // One panel step for 16 columns of one system per workgroup.
 // ---------------------------------------------------------------------------
 
-// One 16 x 16 x 4 matrix-core product.  Lane l = 16 g + q: A operand
-// [q][inner g], B operand [inner g][q], result register e holds row row(g, e)
-// and column q.  Where the inner index of a product is the row index of an
-// earlier result, step e takes inner indices row(0..3, e), so that register e
-// of that result is the B operand as it stands.
-template <typename T>
-struct QrMma;
-template <>
-struct QrMma<float> {
-  typedef float acc __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ acc mul(float a, float b, acc c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ constexpr int row(int g, int e) { return 4 * g + e; }
-};
-template <>
-struct QrMma<double> {
-  typedef double acc __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ acc mul(double a, double b, acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ constexpr int row(int g, int e) { return g + 4 * e; }
-};
+// Where the inner index of a product (Mma) is the row index of an earlier
+// result, step e takes inner indices row(0..3, e), so that register e of that
+// result is the B operand as it stands.
 
 // The 64-bit move (one instruction instead of two); the builtin takes 64-bit
 // values only with literal controls, hence the switch (j is a constant).
@@ -148,7 +128,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
   constexpr int NB = QrCfg<T>::NB;
   static_assert(NB == 16 && KR % 4 == 0, "16-column panels; slots go in groups of four");
   constexpr int kWaves = kPanelWaves, kSpan = 16 * kWaves;  // rows per slot over the waves
-  using M4 = typename QrMma<T>::acc;
+  using M4 = typename Mma<T>::acc;
   extern __shared__ __align__(16) unsigned char step_smem[];
   T* far_slots = reinterpret_cast<T*>(step_smem);  // [KL][4][kPanelThreads]
   __shared__ T s_w[kWaves][NB][NB + 1];
@@ -186,7 +166,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
   int64_t off[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    rel[e] = 16 * wv + QrMma<T>::row(g, e);
+    rel[e] = 16 * wv + Mma<T>::row(g, e);
     off[e] = (int64_t)rel[e] * lda;
   }
   auto base = [&](int s) { return A + (int64_t)min(k + kSpan * s, m - 1) * lda; };  // uniform
@@ -197,7 +177,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
   if (mode != kStepPanel) {
     const T* Tp = tblk + d.t_offset + (int64_t)(k / NB) * NB * NB;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) tt[e] = Tp[QrMma<T>::row(g, e) * NB + q];
+    for (int e = 0; e < 4; ++e) tt[e] = Tp[Mma<T>::row(g, e) * NB + q];
   }
   auto project_v = [&](int s, T (&x)[4]) {
     const T* p = base(s) + k + min(q, nb - 1);
@@ -214,10 +194,10 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
     const T* p = base(s) + (in ? offq : 0) + k;
     T v[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = p[min(QrMma<T>::row(g, e), nb - 1)];
+    for (int e = 0; e < 4; ++e) v[e] = p[min(Mma<T>::row(g, e), nb - 1)];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int j = QrMma<T>::row(g, e);
+      const int j = Mma<T>::row(g, e);
       x[e] = in && j < nb ? -vpick(kSpan * s + rq, j, v[e]) : T(0);
     }
   };
@@ -245,12 +225,12 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int u = 0; u < kWideTiles; ++u) w[u] = QrMma<T>::mul(x[e], exists(s, e) ? c[u][e] : T(0), w[u]);
+        for (int u = 0; u < kWideTiles; ++u) w[u] = Mma<T>::mul(x[e], exists(s, e) ? c[u][e] : T(0), w[u]);
     }
 #pragma unroll
     for (int u = 0; u < kWideTiles; ++u)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s_wide[wv][QrMma<T>::row(g, e)][16 * u + q] = w[u][e];
+      for (int e = 0; e < 4; ++e) s_wide[wv][Mma<T>::row(g, e)][16 * u + q] = w[u][e];
     __syncthreads();
     M4 tw[kWideTiles];
 #pragma unroll
@@ -259,12 +239,12 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
       for (int e = 0; e < 4; ++e) {
         T x = T(0);
 #pragma unroll
-        for (int i = 0; i < kWaves; ++i) x += s_wide[i][QrMma<T>::row(g, e)][16 * u + q];
+        for (int i = 0; i < kWaves; ++i) x += s_wide[i][Mma<T>::row(g, e)][16 * u + q];
         w[u][e] = x;
       }
       tw[u] = M4{T(0), T(0), T(0), T(0)};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) tw[u] = QrMma<T>::mul(tt[e], w[u][e], tw[u]);
+      for (int e = 0; e < 4; ++e) tw[u] = Mma<T>::mul(tt[e], w[u][e], tw[u]);
     }
 #pragma unroll 2
     for (int s = 0; s < ns; ++s) {
@@ -275,7 +255,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int u = 0; u < kWideTiles; ++u) c[u] = QrMma<T>::mul(x[e], tw[u][e], c[u]);
+        for (int u = 0; u < kWideTiles; ++u) c[u] = Mma<T>::mul(x[e], tw[u][e], c[u]);
       T* p = base(s);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -345,27 +325,27 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
       T x[4];
       project_v(s, x);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) w = QrMma<T>::mul(x[e], c[e], w);
+      for (int e = 0; e < 4; ++e) w = Mma<T>::mul(x[e], c[e], w);
     });
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s_w[wv][QrMma<T>::row(g, e)][q] = w[e];
+    for (int e = 0; e < 4; ++e) s_w[wv][Mma<T>::row(g, e)][q] = w[e];
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       T x = T(0);
 #pragma unroll
-      for (int i = 0; i < kWaves; ++i) x += s_w[i][QrMma<T>::row(g, e)][q];
+      for (int i = 0; i < kWaves; ++i) x += s_w[i][Mma<T>::row(g, e)][q];
       w[e] = x;
     }
     // ---- T^T W, then C - V (T^T W)
     M4 tw = {T(0), T(0), T(0), T(0)};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) tw = QrMma<T>::mul(tt[e], w[e], tw);
+    for (int e = 0; e < 4; ++e) tw = Mma<T>::mul(tt[e], w[e], tw);
     each([&](int s, M4& c) __attribute__((always_inline)) {
       T x[4];
       expand_v(s, x);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) c = QrMma<T>::mul(x[e], tw[e], c);
+      for (int e = 0; e < 4; ++e) c = Mma<T>::mul(x[e], tw[e], c);
     });
   }
   if constexpr (KR > 0) {
@@ -390,7 +370,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
         M4 y = v;
         if (s == 0 && wv == t0) {       // uniform: rows above the diagonal and on it stay out
 #pragma unroll
-          for (int e = 0; e < 4; ++e) y[e] = QrMma<T>::row(g, e) > j ? v[e] : T(0);
+          for (int e = 0; e < 4; ++e) y[e] = Mma<T>::row(g, e) > j ? v[e] : T(0);
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -445,7 +425,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const T moved = fma(row_bcast<j>(v[e]), coef, v[e]);
-            v[e] = QrMma<T>::row(g, e) > j ? moved : v[e];
+            v[e] = Mma<T>::row(g, e) > j ? moved : v[e];
           }
           if (g == gj) acc[0][ej] = q == j ? beta : acc[0][ej] + on_diag;
           return;
@@ -458,7 +438,7 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
     each([&](int s, M4& v) __attribute__((always_inline)) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const bool below = s > 0 || wv > t0 || (wv == t0 && QrMma<T>::row(g, e) > q);
+        const bool below = s > 0 || wv > t0 || (wv == t0 && Mma<T>::row(g, e) > q);
         v[e] = below ? v[e] * sc : v[e];
       }
       store(s, v);
@@ -471,11 +451,11 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
         for (int e = 0; e < 4; ++e) {
           const int r = kSpan * s + rel[e] - 16 * t0;
           const T x = q < nbn ? vpick(r, q, v[e]) : T(0);
-          w = QrMma<T>::mul(x, x, w);
+          w = Mma<T>::mul(x, x, w);
         }
       });
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s_w[wv][QrMma<T>::row(g, e)][q] = w[e];
+      for (int e = 0; e < 4; ++e) s_w[wv][Mma<T>::row(g, e)][q] = w[e];
       __syncthreads();
       if (tid < NB * NB) {
         T x = T(0);
