@@ -83,17 +83,16 @@ __device__ __forceinline__ void reflector(double alpha, double ss, double& beta,
   }
 }
 
-// Whether v_q^T v_j may be formed as scales of v_q and v_j times a sum over the
-// unscaled columns (larft in qr_step_kernel): the sum's products, of which
-// there are at most 2^12 with norms below 1 / |sq| and 1 / |sj|, neither
-// overflow nor lose more than rounding to the smallest normal number.
-__device__ __forceinline__ bool unscaled_sums(float sq, float sj) {
-  const float p = fabsf(sq * sj);
-  return p >= 0x1p-100f && p <= 0x1p80f && fabsf(sq) <= 0x1p100f;
+// Whether v_q^T v_j may be formed as the scales of v_q and v_j times a sum over
+// the unscaled columns (larft in qr_step_kernel).  The sum has at most 2^12
+// products and the columns' norms are below 1 / |scale|: with both scales in
+// this range nothing overflows, and what is lost below the smallest normal
+// number is below rounding.
+__device__ __forceinline__ bool unscaled_sums(float scale) {
+  return fabsf(scale) >= 0x1p-50f && fabsf(scale) <= 0x1p40f;
 }
-__device__ __forceinline__ bool unscaled_sums(double sq, double sj) {
-  const double p = fabs(sq * sj);
-  return p >= 0x1p-960 && p <= 0x1p900 && fabs(sq) <= 0x1p960;
+__device__ __forceinline__ bool unscaled_sums(double scale) {
+  return fabs(scale) >= 0x1p-480 && fabs(scale) <= 0x1p450;
 }
 
 // Columns of a workgroup that does not keep them in registers: V is read once
@@ -357,7 +356,6 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
     const int nbn = min(NB, kmax - kn);
     const int t0 = (kn - k) / 16;  // tile with the panel's diagonal: slot 0 of wave t0
     T sc = T(1);                   // scaling of this lane's column below its diagonal, applied when stored
-    bool rescale = false;          // products of this lane's column with a later one are out of range
     static_for<0, NB>([&](auto J_) __attribute__((always_inline)) {
       constexpr int j = decltype(J_)::value;
       if (j >= nbn) return;  // uniform
@@ -410,7 +408,6 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
       }
       // v = [1; scale x]: v^T (column q) for q > j (larf), v_q^T v for q < j
       // (larft; columns left of j are still unscaled)
-      rescale = rescale || (ss != 0.0 && q < j && !unscaled_sums(sc, scale));
       const T prod = dv + scale * dots;
       if (tid < j) s_g[tid][j] = sc * prod;
       if (tid == j) s_tau[j] = tj;
@@ -443,8 +440,9 @@ __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_des
       }
       store(s, v);
     });
-    if (__any(rescale)) {  // uniform over the workgroup: every wave holds all columns' scales
+    if (__any(!unscaled_sums(sc))) {  // uniform over the workgroup: every wave holds all columns' scales
       // ---- V^T V from the scaled columns: a result register is both operands
+      // (1 % of the factor's time at 256 x 512 x 256 in float, 7 % at 4000 x 400)
       M4 w = {T(0), T(0), T(0), T(0)};
       each_read([&](int s, const M4& v) __attribute__((always_inline)) {
 #pragma unroll
