@@ -225,8 +225,6 @@ __device__ void wave_chol_solve(int n, const T* L, T (&v)[4]) {
     rd[c] = T(1) / d[c];
     plain = plain && plain_range(d[c]);
   }
-  const bool fast = __all(plain);
-  auto over = [&](T x, int c) { return fast ? divide(x, d[c], rd[c]) : x / d[c]; };
   // U^T y = v, column oriented: y_k = v_k / U_kk, then v_j -= U_kj y_k.
   auto row = [&](int k, T (&to)[4]) {
     const int kc = min(k, n - 1);
@@ -234,45 +232,68 @@ __device__ void wave_chol_solve(int n, const T* L, T (&v)[4]) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) to[c] = R[max(min(l + 64 * c, n - 1), kc)];
   };
-  T cur[4], nxt[4];
-  row(0, nxt);
-#pragma unroll
-  for (int c0 = 0; c0 < 4; ++c0) {
-    const int kend = min(64, n - 64 * c0);
-    for (int kk = 0; kk < kend; ++kk) {
-      const int k = 64 * c0 + kk;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) cur[c] = nxt[c];
-      row(k + 1, nxt);
-      const T yk = from_lane(over(v[c0], c0), kk);
-      if (l == kk) v[c0] = yk;
-#pragma unroll
-      for (int c = c0; c < 4; ++c)
-        if (l + 64 * c > k) v[c] -= cur[c] * yk;
-    }
-  }
   // U x = y, column oriented: x_k = y_k / U_kk, then y_i -= U_ik x_k.
   auto column = [&](int k, T (&to)[4]) {
     const int kc = max(k, 0);
 #pragma unroll
     for (int c = 0; c < 4; ++c) to[c] = L[packed_upper(n, min(l + 64 * c, kc), kc)];
   };
-  column(n - 1, nxt);
+  auto sweeps = [&](auto Fast_) __attribute__((always_inline)) {
+    auto over = [&](T x, int c) {
+      if constexpr (decltype(Fast_)::value) {
+        return divide(x, d[c], rd[c]);
+      } else {
+        return x / d[c];
+      }
+    };
+    T cur[4], nxt[4];
+    row(0, nxt);
 #pragma unroll
-  for (int c0 = 3; c0 >= 0; --c0) {
-    const int kend = min(64, n - 64 * c0);
-    for (int kk = kend - 1; kk >= 0; --kk) {
-      const int k = 64 * c0 + kk;
+    for (int c0 = 0; c0 < 4; ++c0) {
+      const int kend = min(64, n - 64 * c0);
+      for (int kk = 0; kk < kend; ++kk) {
+        const int k = 64 * c0 + kk;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) cur[c] = nxt[c];
-      column(k - 1, nxt);
-      const T xk = from_lane(over(v[c0], c0), kk);
-      if (l == kk) v[c0] = xk;
+        for (int c = 0; c < 4; ++c) cur[c] = nxt[c];
+        row(k + 1, nxt);
+        const T yk = from_lane(over(v[c0], c0), kk);
+        if (l == kk) v[c0] = yk;
 #pragma unroll
-      for (int c = 0; c <= c0; ++c)
-        if (l + 64 * c < k) v[c] -= cur[c] * xk;
+        for (int c = c0; c < 4; ++c)
+          if (l + 64 * c > k) v[c] -= cur[c] * yk;
+      }
     }
+    column(n - 1, nxt);
+#pragma unroll
+    for (int c0 = 3; c0 >= 0; --c0) {
+      const int kend = min(64, n - 64 * c0);
+      for (int kk = kend - 1; kk >= 0; --kk) {
+        const int k = 64 * c0 + kk;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) cur[c] = nxt[c];
+        column(k - 1, nxt);
+        const T xk = from_lane(over(v[c0], c0), kk);
+        if (l == kk) v[c0] = xk;
+#pragma unroll
+        for (int c = 0; c <= c0; ++c)
+          if (l + 64 * c < k) v[c] -= cur[c] * xk;
+      }
+    }
+  };
+  if (__all(plain)) {
+    T b[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) b[c] = v[c];
+    sweeps(std::true_type{});
+    bool again = false;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) again = again || (l + 64 * c < n && v[c] != v[c]);
+    if (!__any(again)) return;
+    // NaN may be an infinite quotient: once more with divisions
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] = b[c];
   }
+  sweeps(std::false_type{});
 }
 
 template <typename T>

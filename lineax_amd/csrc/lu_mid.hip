@@ -310,7 +310,7 @@ __global__ __launch_bounds__(kSolveThreads) void lu_mid_solve_kernel(int n, cons
     __syncthreads();
   }
   const T rdiag = T(1) / diag;
-  const bool fast = __all(plain_range(diag));
+  bool fast = __all(plain_range(diag));
 
   // entries that couple unknown i to the 16 unknowns of block p
   auto fetch = [&](int p, T (&v)[kP]) {
@@ -353,20 +353,28 @@ __global__ __launch_bounds__(kSolveThreads) void lu_mid_solve_kernel(int n, cons
   };
   using Yes = std::true_type;
   using No = std::false_type;
-  if (!trans) {
-    sweep(Yes{}, No{});   // L y = P b
-    sweep(No{}, Yes{});   // U x = y
-    if (in) B[i] = y;
-  } else {
-    sweep(Yes{}, Yes{});  // U^T z = b
-    sweep(No{}, No{});    // L^T w = z
-    int p = i;
+  const T rhs = y;
+  while (true) {
+    if (!trans) {
+      sweep(Yes{}, No{});   // L y = P b
+      sweep(No{}, Yes{});   // U x = y
+    } else {
+      sweep(Yes{}, Yes{});  // U^T z = b
+      sweep(No{}, No{});    // L^T w = z
+    }
+    // NaN may be an infinite quotient: once more with divisions
+    if (!__syncthreads_or(fast && in && y != y)) break;
+    fast = false;
+    y = rhs;
+  }
+  int p = i;
+  if (trans) {
     for (int k = n - 1; k >= 0; --k) {
       const int o = pv[k];
       p = (p == k) ? o : ((p == o) ? k : p);
     }
-    if (in) B[p] = y;     // every read of B is behind the barriers above
   }
+  if (in) B[p] = y;  // every read of B is behind the barriers above
 }
 
 template <typename T, int S, bool InLds>

@@ -5,7 +5,6 @@
 
 #include <cmath>
 #include <cstdint>
-#include <limits>
 #include <type_traits>
 
 #include "../../include/lineax_amd.h"
@@ -214,12 +213,12 @@ __device__ __forceinline__ R wave_reduce_scatter(R (&v)[K], int lane) {
 __device__ __forceinline__ bool plain_range(float d) { return fabsf(d) >= 0x1p-100f && fabsf(d) <= 0x1p100f; }
 __device__ __forceinline__ bool plain_range(double d) { return fabs(d) >= 0x1p-900 && fabs(d) <= 0x1p900; }
 
+// An infinite quotient comes out as NaN (its correction is inf - inf): callers
+// whose quotients may overflow look for NaN at their end and divide instead.
 template <typename T>
 __device__ __forceinline__ T divide(T x, T d, T rd) {
   const T q = x * rd;
-  const T c = fma(fma(-d, q, x), rd, q);
-  // an infinite quotient has no correction (it would be inf - inf)
-  return fabs(q) <= std::numeric_limits<T>::max() ? c : q;
+  return fma(fma(-d, q, x), rd, q);
 }
 
 // Index of element (i, j), j >= i, in a row-packed upper triangle of order n.
