@@ -398,7 +398,7 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
   T* ys = reinterpret_cast<T*>(lxa_smem);  // [n rounded up to R]
   __shared__ T part[kSolveWaves][R];
   __shared__ T D[2][R][R + 1];            // diagonal blocks, double-buffered
-  __shared__ T rd[2][R];                  // reciprocals of their diagonals
+  __shared__ T rd[2][R];                  // reciprocals of their diagonals, 0 where that is no normal number
   const T* U = u + (int64_t)blockIdx.x * u_stride;
   T* B = b + (int64_t)blockIdx.x * b_stride;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -442,7 +442,7 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
       if (di < R) {
         const bool in = p * R + dj < n && dj >= di;
         D[p & 1][di][dj] = in ? dv[h] : T(0);
-        if (di == dj) rd[p & 1][di] = in ? T(1) / dv[h] : T(0);  // padding solves to 0
+        if (di == dj) rd[p & 1][di] = in && plain_range(dv[h]) ? T(1) / dv[h] : T(0);  // padding solves to 0
       }
     }
   };
@@ -478,11 +478,12 @@ __global__ __launch_bounds__(kSolveThreads) void chol_tile_solve_kernel(int n, c
   // as divisions where one of the block's entries has none that is normal
   // (never a factor of lxa_chol_factor, whose entries are square roots)
   auto chain = [&](int p, auto&& f) __attribute__((always_inline)) {
-    const T d = D[p & 1][lane % R][lane % R], r = rd[p & 1][lane % R];
+    const T r = rd[p & 1][lane % R];
     const bool pad = p * R + lane % R >= n;
-    if (__all(pad || plain_range(d))) {
+    if (__all(pad || r != T(0))) {
       f([&](T z) { return z * r; });
     } else {
+      const T d = D[p & 1][lane % R][lane % R];
       f([&](T z) { return pad ? T(0) : z / d; });
     }
   };
