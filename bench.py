@@ -356,7 +356,8 @@ def bench_uneven_cholesky(args):
             "p50_ms": _percentile(pms, 50),
             "p99_ms": _percentile(pms, 99),
             "kernels": "lxa_chol_factor + lxa_chol_solve per order bucket (the lx.Cholesky path)",
-            "launches_per_step": 2 * len(batch.buckets),
+            # a factor and a solve; past order 64 the factor is a launch per 64 columns and one for failures
+            "launches_per_step": sum(2 if n <= 64 else 2 + (n + 63) // 64 for n, _, _ in batch.buckets),
             "max_backward_error_sample": eta_sample(lambda i: where[int(i)]),
             "x_dtype": "float32",
             "achieved_gbs": batch.algorithmic_bytes / (float(np.mean(pms)) / 1e3) / 1e9,

@@ -12,7 +12,7 @@
 //            the product with the inverse of the unit lower 16 x 16 block.
 //   update   A22 -= L21 U12 in 16 x 16 tiles on the matrix cores, the type's
 //            own products and sums.
-// The matrix stays in LDS where it fits (order 200 in float, 141 in double);
+// The matrix stays in LDS where it fits (order 199 in float, 141 in double);
 // above that it stays in global memory (L2) with L21 and U12 staged in LDS.
 // The result is getrf's: factors in place, 0-based interchange sequence, info
 // the first exactly zero pivot.

@@ -18,8 +18,8 @@
 // Panels taller than 4096 rows are factored from global memory by
 // qr_panel_kernel and updated in two sweeps over C.
 //
-// The panel's chain of columns bounds single and small batches (28 us a panel
-// at up to 512 rows, 63 us at 3001 double rows, 80 us at 4096 float rows, one
+// The panel's chain of columns bounds single and small batches (29 us a panel
+// at up to 512 rows, 64 us at 3001 double rows, 76 us at 4000 float rows, one
 // barrier and two passes over the registers a column), HBM the large ones.  With a
 // launch each for panel, partial products, their sum and the update, 256
 // float systems of 512 x 256 took 1490 us; they take 940 us here.

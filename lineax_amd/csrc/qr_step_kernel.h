@@ -115,8 +115,9 @@ inline int step_blocks(int KR, int mode, int right) {
 }
 
 // KR: 16-row tiles per wave held in registers (slot s of wave w is tile
-// w + 8 s of the rows from k on); KL: further ones in LDS (the register file
-// holds 2048 double or 3072 float rows beside what the products need).
+// w + 8 s of the rows from k on); KL: further ones in LDS (28 slots, 3584 rows,
+// in float and 24, 3072 rows, in double are what 256 registers hold beside the
+// products' operands, the 24 with a few dozen bytes of scratch a lane).
 // KR = 0: wide blocks only, any height.
 template <typename T, int KR, int KL>
 __global__ __launch_bounds__(kPanelThreads) void qr_step_kernel(const lxa_qr_desc* __restrict__ descs, int64_t count,
